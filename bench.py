@@ -234,8 +234,8 @@ def stage_rooflines(spec, path, n_exact):
         add("taylor", "k_taylor (5 complex V t products, FP64 MFMA)", Wp * 40.0 * N * N * ncol, tay_bytes, 5,
             "fp64", symbol=("void k_taylor<%s>" % ("true" if N % 2 == 0 else "false")) if wide
             else "void k_vmul<64, 128, 2, 2>")
-        add("force_bias", "k_force_bias (FP64 MFMA)", Wl * 4.0 * ncol * N * G, 8.0 * G * ms + Wl * 16.0 * (ms + G),
-            1, "fp64", symbol="k_force_bias")
+        add("force_bias", "k_fb64 (FP64 MFMA)", Wl * 4.0 * ncol * N * G, 8.0 * G * ms + Wl * 16.0 * (ms + G),
+            1, "fp64", symbol="k_fb64")
         add("vhs", "k_vhs (FP64 MFMA)", Wp * 4.0 * T * G, 8.0 * G * T + Wp * 16.0 * (G + N * N), 1, "fp64",
             symbol="k_vhs")
     else:

@@ -19,11 +19,11 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libvmc_afqmc.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
-SOURCES = ["afq_kernels.hip", "afq_exchange_pw2.hip", "afq_exchange_pw2x3.hip", "afq_mlp.hip", "afq_ctx.cpp", "afq_driver.cpp",
+SOURCES = ["afq_kernels.hip", "afq_force_bias.hip", "afq_exchange_pw2.hip", "afq_exchange_pw2x3.hip", "afq_mlp.hip", "afq_ctx.cpp", "afq_driver.cpp",
            "afq_noalloc.cpp"]
 # per-file hipcc options: the pair-wise exchange keeps its MFMA accumulators in VGPRs
 SOURCE_FLAGS = {"afq_exchange_pw2.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-HEADERS = ["afq_device.hpp", "afq_internal.hpp", "afq_group.hpp", "afq_exchange_pw2.hpp"]
+HEADERS = ["afq_device.hpp", "afq_internal.hpp", "afq_group.hpp", "afq_exchange_pw2.hpp", "afq_gemm64.hpp"]
 CPP_TESTS = [("tests/cpp/api_parity.cpp", "tests/cpp/api_parity")]  # host programs over the C++ mirror
 # FCIDUMP_chol (HDF5) reader/writer, a host library of its own: built where the HDF5 C
 # library is installed (HDF5_DIR, default /opt/conda), skipped otherwise

@@ -295,6 +295,9 @@ void alloc_walkers(DevState& s) {
   s.draws = dalloc<double>(W * s.G);
   s.Xp = dalloc<double>(2 * (int64_t)s.nslots * W * s.ngt_cap);
   s.Sg = dalloc<double>((int64_t)W * s.nslots * 64 * 128);
+  const bool big = W * s.nslots * 64 * 128 >= 2 * W * s.Ktot;
+  s.fbw = big ? s.Sg : s.theta2;
+  s.fbw_doubles = big ? W * s.nslots * 64 * 128 : 2 * W * s.Ktot;
   s.eloc = dalloc<double>(W);
   s.ho = dalloc<double>(4 * W);
   s.cum = dalloc<double>(W);
@@ -1030,6 +1033,8 @@ int afq_ham_and_overlap(afq_ctx* c, const double* dets, int32_t ndet, int32_t nc
   t.W = ndet;
   t.GE = nchol_ene;
   alloc_walkers(t);
+  t.fbw = t.Sg;
+  t.fbw_doubles = (int64_t)ndet * t.nslots * 64 * 128;
   try {
     upload(t.psi, dets, 2 * (size_t)ndet * t.ms, c->stream);
     afq::launch_fill(t.weights, ndet, 1.0, c->stream);

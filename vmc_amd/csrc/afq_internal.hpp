@@ -86,6 +86,12 @@ struct DevState {
   double* t0 = nullptr; double* t1 = nullptr; double* accb = nullptr;  // W x ms complex
   double* draws = nullptr;   // W x G (replay)
   double* Sg = nullptr;      // W x nslots x 64 x 128: overlap matrices S = Phi^T psi, then S^-1
+  // FP64 force bias: partial sums over chunks of K.  Not a buffer of its own: it borrows
+  // one that nothing reads between the Green's function and the end of the force bias,
+  // the larger of Sg (S^-1 is used up by theta) and theta2 (live inside a comb only);
+  // a temporary population borrows Sg, whichever entry point made it, so that all of
+  // them split K alike
+  double* fbw = nullptr; int64_t fbw_doubles = 0;
   double* Xp = nullptr;      // nslots x W x ngt complex exchange partials
   int ngt_cap = 0;
   double* eloc = nullptr;    // W
@@ -234,7 +240,11 @@ void launch_risk_split(const DevState& s, const double* ej, double risk, RiskSor
                        hipStream_t st);
 
 // kernel launchers (afq_kernels.hip)
-void launch_force_bias(const DevState& s, hipStream_t st);
+void launch_force_bias(const DevState& s, hipStream_t st);   // afq_force_bias.hip
+// the split of the FP64 force bias of W walkers: the 32 x 64 or the 64 x 64 tile, and
+// nz chunks of kchunk (a multiple of 16) of the Ktot products
+struct FbPlan { bool small; int nz, kchunk; };
+FbPlan fb_plan(int W, int G, int64_t Ktot, int64_t ws_doubles);
 void launch_fields(const DevState& s, const double* draws, uint64_t seed, uint64_t step, hipStream_t st);
 void launch_vhs(const DevState& s, hipStream_t st);
 void launch_propagate(const DevState& s, hipStream_t st);  // E psi, Taylor terms, E acc

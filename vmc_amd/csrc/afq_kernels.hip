@@ -2,7 +2,6 @@
 //
 // Every dense contraction is a real GEMM on the FP64 MFMA tile engine
 // (afq_device.hpp) with loaders that read the operand in its storage layout:
-//   force bias    C[(w,c), g]  = sum_k theta[w][k][c] R[g][k]          (DQMC/RHF.cpp:54-61, DQMC/UHF.cpp:45-53)
 //   VHS           P[(w,c), t]  = sum_g field[w][g][c] Lp[g][t]          (DQMC/DQMCWalker.cpp:406-421)
 //   one-body      E psi, batched over walkers folded into columns        (DQMC/DQMCWalker.cpp:482-491)
 //   Taylor term   V t with complex V embedded as [A_re | A_im] x [[B_re,B_im],[-B_im,B_re]]
@@ -23,60 +22,6 @@
 namespace afq {
 
 static inline unsigned cdivu(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
-
-// ------------------------------------------------------------------ force bias
-struct FbA {  // A((l,c), k) = theta[w][k][c] for the l-th live walker w = live[l]
-  const double* th; const int* live; int64_t Ktot; int row0, nrow;
-  __device__ double operator()(int r, int k) const {
-    const int q = row0 + r;
-    if (q >= nrow || k >= Ktot) return 0.0;
-    return th[(int64_t)live[q >> 1] * 2 * Ktot + 2 * (int64_t)k + (q & 1)];
-  }
-};
-struct FbB {  // B(k, g) = R[g][k]
-  const double* R; int64_t Ktot; int g0, G;
-  __device__ double operator()(int k, int c) const {
-    const int g = g0 + c;
-    if (g >= G || k >= Ktot) return 0.0;
-    return R[(int64_t)g * Ktot + k];
-  }
-};
-
-constexpr int FB_BM = 128, FB_BN = 128;
-// Force bias of the walkers with nonzero weight only (live[0 .. *nlive)): a walker of
-// weight zero is neither propagated nor measured (DQMC/MixedEstimator.cpp:461-468,531)
-// and the comb replaces it, so its force bias is never read.  (A walker below the
-// propagation threshold 1e-8 but nonzero is still measured, and E_J needs its force
-// bias.)  The grid covers every walker; tiles past the live count exit.
-__device__ __forceinline__ void k_force_bias_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* th, double* fb,
-                                                    const int* live, const int* nlive, int G, int64_t Ktot,
-                                                    double alpha, int gridx, int gridy) {
-  using Eng = MmaF64<FB_BM, FB_BN, 2, 2, false, false>;
-  __shared__ double lds[Eng::LDS_DOUBLES];
-  const TileId tl = tile_id_at(bid_.x, gridx, gridy, 1, 8);
-  const int row0 = tl.y * FB_BM, g0 = tl.x * FB_BN;
-  const int nrow = 2 * *nlive;
-  if (row0 >= nrow) return;
-  Eng e;
-  e.run(FbA{th, live, Ktot, row0, nrow}, FbB{R, Ktot, g0, G}, (int)Ktot, lds);
-  e.store([&](int r, int c, double v) {
-    const int q = row0 + r, g = g0 + c;
-    if (q < nrow && g < G) fb[(int64_t)live[q >> 1] * 2 * G + 2 * g + (q & 1)] = alpha * v;
-  });
-}
-struct F_k_force_bias {
-  static constexpr int NT = 256, OCC = 2;
-  static constexpr bool HAS_OCC = true;
-  template <class... A>
-  __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_force_bias_body(b, g, a...);
-  }
-};
-__global__ __launch_bounds__(256, 2) void k_force_bias(const double* R, const double* th, double* fb,
-                                                    const int* live, const int* nlive, int G, int64_t Ktot,
-                                                    double alpha, int gridx, int gridy) {
-  k_force_bias_body(blockIdx3(), gridDim3(), R, th, fb, live, nlive, G, Ktot, alpha, gridx, gridy);
-}
 
 // live[0 .. *count) = the walkers of nonzero weight, ascending (one workgroup)
 __device__ __forceinline__ void k_live_list_body(const uint3 bid_, const uint3 gdim_, const double* weights, int W, int* live, int* count) {
@@ -114,13 +59,6 @@ __global__ __launch_bounds__(1024) void k_live_list(const double* weights, int W
 }
 void launch_live_list(const DevState& s, hipStream_t st) {
   afq::glaunch<F_k_live_list>(k_live_list, dim3(1), dim3(1024), 0, st, s.weights, s.W, s.live, s.nlive);
-}
-
-void launch_force_bias(const DevState& s, hipStream_t st) {
-  launch_live_list(s, st);
-  const int gx = (int)cdivu(s.G, FB_BN), gy = (int)cdivu(2 * (int64_t)s.W, FB_BM);
-  afq::glaunch<F_k_force_bias>(k_force_bias, dim3(gx * gy), dim3(256), 0, st, s.R, s.theta, s.fb, s.live, s.nlive, s.G, s.Ktot,
-                     (double)s.slot[0].mult, gx, gy);
 }
 
 // ------------------------------------------------------------------ fields
@@ -3375,7 +3313,7 @@ __device__ __forceinline__ void k_force_bias_bf16_body(const uint3 bid_, const u
   __shared__ __attribute__((aligned(16))) unsigned char lds[Eng::LDS_BYTES];
   const TileId tl = tile_id_at(bid_.x, gridx, gridy, part ? nslots : 1, 8);
   const int row0 = tl.y * 128, g0 = tl.x * 128;
-  const int nrow = 2 * *nlive;   // live walkers only, as k_force_bias
+  const int nrow = 2 * *nlive;   // live walkers only, as the FP64 force bias
   if (row0 >= nrow) return;
   Eng e;
   int64_t roff = 0;

@@ -81,6 +81,8 @@ void carve_population(afq::DevState& t, int ndet, Carve& c) {
   t.logdet = c.take<double>(2 * n * t.nslots);
   t.weights = c.take<double>(n);
   t.Sg = c.take<double>(n * t.nslots * 64 * 128);
+  t.fbw = t.Sg;
+  t.fbw_doubles = n * t.nslots * 64 * 128;
   t.Xp = c.take<double>(2 * (int64_t)t.nslots * n * t.ngt_cap);
   t.eloc = c.take<double>(n);
   t.ho = c.take<double>(4 * n);
