@@ -1734,8 +1734,9 @@ int afq_sync(afq_ctx* c) {
 // ---------------------------------------------------------------- autotuner
 // Times the alternative tile shapes of the Taylor products (k_vmul's 64 x 128 real
 // tiles against k_taylor's 128 x 128-complex tiles) on this context's current
-// walkers and keeps the faster one.  The products only write Taylor scratch, so the
-// walker state is unchanged.
+// walkers and keeps the faster one; in FP64 the fused k_prop64, where it applies, is kept
+// over both when its whole propagation takes less than their Taylor products alone.  The
+// products only write Taylor scratch, so the walker state is unchanged.
 int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   if (!c) return AFQ_ERR_ARG;
   if (!c->prepped || !c->have_walkers) return fail(c, AFQ_ERR_STATE, "afq_prep_prop and afq_set_walkers first");
@@ -1747,6 +1748,7 @@ int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   double best = 1e300;
   int pick = 1;
   const int keep = s.taylor_variant;
+  bool fused64 = false;
   // split BF16: the whole propagation (both one-body factors and the series) into the
   // scratch t1, so the walkers stay as they are; FP64: the five Taylor products
   const bool split = s.prec_prop != AFQ_PREC_FP64;
@@ -1769,6 +1771,16 @@ int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
       if (ms_out) ms_out[v - 1] = ms / 3.0;
       if (ms < best) { best = ms; pick = v; }
     }
+    if (!split && afq::prop64_fits(s)) {
+      afq::launch_prop64(s, s.t1, c->stream);  // warm
+      hip_check(hipEventRecord(a, c->stream), "record");
+      for (int r = 0; r < 3; ++r) afq::launch_prop64(s, s.t1, c->stream);
+      hip_check(hipEventRecord(b, c->stream), "record");
+      hip_check(hipEventSynchronize(b), "sync");
+      float ms = 0.f;
+      hip_check(hipEventElapsedTime(&ms, a, b), "elapsed");
+      fused64 = ms < best;
+    }
   } catch (...) {
     s.taylor_variant = keep;
     (void)hipEventDestroy(a);
@@ -1777,7 +1789,7 @@ int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   }
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
-  s.taylor_variant = pick;
+  s.taylor_variant = fused64 ? 0 : pick;
   if (choice) *choice = pick;
   return AFQ_OK;
   AFQ_GUARD_END(c)

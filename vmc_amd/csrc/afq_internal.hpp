@@ -152,7 +152,7 @@ struct DevState {
   const double* d_zeta = nullptr;
   bool graph_mode = false;
   // Taylor kernels: 0 by shape; FP64: 1 k_vmul (64 x 128 tiles), 2 k_taylor (128 x 128
-  // complex); split BF16: 1 128-row tiles, 2 160-row tiles (one-body factors and Taylor
+  // complex), both between separate one-body products, else the fused k_prop64 (N <= 384); split BF16: 1 128-row tiles, 2 160-row tiles (one-body factors and Taylor
   // steps as separate kernels), 3 the fused k_prop_split (the default where N <= 384)
   int taylor_variant = 0;
   // one-pass BF16 exchange: 0 by shape (k_exchange_pw2 with 8 waves where it applies,
@@ -252,6 +252,8 @@ void launch_expmul_pre(const DevState& s, hipStream_t st);
 void launch_taylor(const DevState& s, hipStream_t st);
 void launch_expmul_post(const DevState& s, hipStream_t st);
 bool prop_fused_fits(const DevState& s);                              // k_prop_split handles N
+bool prop64_fits(const DevState& s);                                  // k_prop64 handles N (afq_prop64.hip)
+void launch_prop64(const DevState& s, double* dst, hipStream_t st);   // the fused FP64 propagation, result in dst
 void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st);  // split path, result in dst
 void launch_green(const DevState& s, bool all_walkers, hipStream_t st);
 void launch_green_pre(const DevState& s, bool all_walkers, hipStream_t st);   // S, S^-1, log det S

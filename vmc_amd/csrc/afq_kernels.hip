@@ -1224,8 +1224,13 @@ void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st) {
   launch_onebody_split(s, s.accb, dst, 1, st);
 }
 
+// the fused FP64 propagation (k_prop64) runs in launch_taylor
+static bool prop64(const DevState& s) {
+  return s.prec_prop == AFQ_PREC_FP64 && s.taylor_variant != 1 && s.taylor_variant != 2 && prop64_fits(s);
+}
 // psi <- E (sum_{k<=5} V^k / k!) E psi  for every live walker
 void launch_expmul_pre(const DevState& s, hipStream_t st) {
+  if (prop64(s)) return;
   if (s.prec_prop != AFQ_PREC_FP64) {
     if (!prop_fused(s)) launch_onebody_split(s, s.psi, s.t0, 0, st);
     return;
@@ -1303,6 +1308,10 @@ static void taylor_fp64(const DevState& s, const double* P, int dsel, hipStream_
   }
 }
 void launch_taylor(const DevState& s, hipStream_t st) {
+  if (prop64(s)) {
+    launch_prop64(s, s.psi, st);
+    return;
+  }
   if (s.uints && s.prec_prop == AFQ_PREC_FP64) {
     // unrestricted integrals: each determinant with its own spin's V (DQMC/DQMCWalker.cpp:532-540)
     taylor_fp64(s, s.P, 0, st);
@@ -1341,6 +1350,7 @@ void launch_taylor(const DevState& s, hipStream_t st) {
   }
 }
 void launch_expmul_post(const DevState& s, hipStream_t st) {
+  if (prop64(s)) return;
   if (s.prec_prop != AFQ_PREC_FP64) {
     if (!prop_fused(s)) launch_onebody_split(s, s.accb, s.psi, 1, st);
     return;
