@@ -385,9 +385,10 @@ int afq_set_exchange_variant(afq_ctx* ctx, int32_t variant);
  * walkers take the chunks in the same order, so more chunks keep the rotated Cholesky
  * rows the resident workgroups read within the L2 of their XCD. */
 int afq_set_exchange_chunks(afq_ctx* ctx, int32_t chunks);
-/* FP64 exchange kernel (no counterpart in the reference), 128 x 128 tiles: 0 (default)
- * the pointer-loader engine with double-buffered stages and 8 waves, 1 the element-loader
- * engine (4 waves, two barriers per stage), 2 the pointer-loader engine with 4 waves. */
+/* FP64 exchange kernel (no counterpart in the reference): 0 (default) 64-row x 64-complex-
+ * column tiles whose operands go straight from memory to registers, for slots of at least
+ * 4 electrons (below: as 2); 128 x 128 tiles through LDS: 1 the element-loader engine (two
+ * barriers per stage), 2 the pointer-loader engine (double-buffered stages). */
 int afq_set_exchange64_variant(afq_ctx* ctx, int32_t variant);
 /* Split-BF16 VHS tile (no counterpart in the reference): 0 128 (walker, component) rows
  * by one 16 x 8 block of V, 64-deep single-buffered stages; 1 256 rows, eight waves,

@@ -1,0 +1,255 @@
+// FP64 exchange: Xp[s][w][tile] = sum over a tile of Cholesky vectors g of
+// sum_ij f_ij f_ji, f = R_{s,g} theta_s (DQMC/UHF.cpp:94-100), without writing f to memory.
+#include <algorithm>
+
+#include "afq_device.hpp"
+#include "afq_internal.hpp"
+
+namespace afq {
+
+static inline unsigned cdivu(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
+
+// One workgroup (four waves) takes gt = 64 / n walkers of a slot and a chunk of the
+// Cholesky vectors, gt at a time: the tile's rows are (vector, i), at most 64, its columns
+// (walker, j), at most 64 complex ones, 16 for each wave.  Both operands go from global
+// memory straight into MFMA registers, NS - 1 K steps of 4 ahead: one 16-byte load of a lane
+// holds re and im of a theta column (the B operands of two MFMA tiles), and for even n two
+// rows of R_g (the A operands of two tiles: rows 2 l of 32 in one, 2 l + 1 in the other; for
+// odd n, where a pair of rows may belong to two vectors, two 8-byte loads).  The waves of a
+// workgroup share the R lines in the vector L1, and without staging the K loop has no
+// barrier.  f then goes to LDS and the sum runs over i <= j (off-diagonal pairs count
+// twice), so that every element of f is read once.  A group of tpb threads keeps the same
+// (vector, walker) place of the tile for the whole chunk and accumulates in registers; the
+// chunk's sum goes to the first of the chunk's partials and zeros to the others.
+//
+// Bound by FP64 MFMA issue.  N = 300, 60+60, G = 1200, 256 walkers: 53.4 ms on the 128 x 128
+// LDS-staged kernel before, 47.8 now (56 TFLOP/s useful, 64 with the padding of 60 to 64;
+// 46.0 of it the K loops, timed without the pair sums).  N = 100, 20+20, G = 400, 1024
+// walkers: 3.8 -> 2.86 ms (47 TFLOP/s; K loops 2.54).  A form with LDS stages of both
+// operands took 56 and 3.3 ms (two 8-byte LDS reads per MFMA), one with 8-byte global loads
+// per tile 49.2 and 3.06.  NS = 6 against 4: equal at N = 100 and 300, 3% faster on systems of
+// N = 20 to 120.
+constexpr int X64_LDF = 130;   // 16-byte rows; transposed 16-byte reads of 16 lanes on 64 banks
+constexpr int X64_NT = 256;
+typedef double __attribute__((ext_vector_type(2), aligned(8))) x64_pair;   // two rows of R, 8-byte aligned
+template <bool EVEN>
+__device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* theta,
+                                                  const int* sel, const int* nsel_dev, double* Xp, int N, int GE, int nw,
+                                                  int W, int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
+                                                  int gridx, int gridy, int gridz) {
+  constexpr int NS = 6;
+  __shared__ __attribute__((aligned(16))) double lds[64 * X64_LDF];
+  const TileId tl = tile_id_at(bid_.x, gridx, gridy, gridz, 8);
+  const Slot sl = tl.z == 0 ? s0 : s1;
+  const int n = sl.n, gt = 64 / n, w0 = tl.y * gt, nrow = gt * n;
+  if (nsel_dev) nw = *nsel_dev;
+  if (w0 >= nw) return;
+  const int ga = tl.x * spc * gslot, gb = min(GE, ga + spc * gslot);   // this chunk's vectors
+  const int tid = threadIdx.x, lane = tid & 63, cl = lane & 15, kh = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool busy = 16 * wave < nrow;   // this wave's columns hold data
+  // rows 32 .. nrow (gt n > 32 always): as two tiles, or as one where at most 16 (row 32 + cl)
+  const int rest = nrow - 32;
+  const bool two1 = rest > 16;
+  // A: rows past the data read a valid one
+  auto split = [&](int r, int& g, int& e) {
+    r = min(r, nrow - 1);
+    g = r / n;
+    e = r - g * n;
+  };
+  int ag[2][2], ae[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    split(2 * cl + t, ag[0][t], ae[0][t]);
+    split(two1 ? 32 + min(2 * cl, EVEN ? rest - 2 : rest) + t : 32 + cl, ag[1][t], ae[1][t]);   // an even n's pair stays one
+  }
+  // B: complex column 16 wave + cl = (walker, j); columns past the data read a valid one
+  const double* pb;
+  {
+    const int c = min(16 * wave + cl, nrow - 1), wl = c / n, j = c - wl * n;
+    const int wi = w0 + wl < nw ? w0 + wl : w0;
+    const int w = sel ? sel[wi] : wi;
+    pb = theta + (int64_t)w * 2 * Ktot + 2 * sl.koff + 2 * j;
+  }
+  const double* Rs = R + sl.koff;
+  const int nk = (N + 3) >> 2;
+  const double* pa[2][2];
+  double2 A[NS][2], B[NS];
+  auto rows = [&](int g0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) pa[h][t] = Rs + (int64_t)min(g0 + ag[h][t], GE - 1) * Ktot + ae[h][t];
+  };
+  auto load = [&](int s, int set) {
+    const int k = min(4 * s + kh, N - 1);
+    auto two = [&](int h) {
+      if (EVEN) {
+        const x64_pair v = *reinterpret_cast<const x64_pair*>(pa[h][0] + k * n);
+        A[set][h] = double2{v.x, v.y};
+      } else {
+        A[set][h].x = pa[h][0][k * n];
+        A[set][h].y = pa[h][1][k * n];
+      }
+    };
+    two(0);
+    if (two1) two(1);
+    else A[set][1].x = pa[1][0][k * n];
+    B[set] = *reinterpret_cast<const double2*>(pb + k * 2 * n);
+  };
+  f64x4 acc[2][2][2];   // [32 rows][even, odd][re, im]
+  auto step = [&](int set) {
+    if (!busy) return;
+    acc[0][0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][0].x, B[set].x, acc[0][0][0], 0, 0, 0);
+    acc[0][0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][0].x, B[set].y, acc[0][0][1], 0, 0, 0);
+    acc[0][1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][0].y, B[set].x, acc[0][1][0], 0, 0, 0);
+    acc[0][1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][0].y, B[set].y, acc[0][1][1], 0, 0, 0);
+    acc[1][0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][1].x, B[set].x, acc[1][0][0], 0, 0, 0);
+    acc[1][0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][1].x, B[set].y, acc[1][0][1], 0, 0, 0);
+    if (two1) {
+      acc[1][1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][1].y, B[set].x, acc[1][1][0], 0, 0, 0);
+      acc[1][1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[set][1].y, B[set].y, acc[1][1][1], 0, 0, 0);
+    }
+  };
+  // pair sums: threads [b tpb, (b + 1) tpb) take block b = (vector b / gt, walker b % gt) of a tile
+  const int tpb = X64_NT / (gt * gt);
+  const int blk = tid / tpb, lt = tid - blk * tpb, pg = blk / gt, pw = blk - pg * gt;
+  // units (p, t): rows p and n - 1 - p share the n + 1 pairs i <= j
+  const int np = (n + 1) >> 1, sp = tpb / (n + 1), stt = tpb - sp * (n + 1);
+  double accr = 0.0, acci = 0.0;
+  rows(ga);
+#pragma unroll
+  for (int i = 0; i + 1 < NS; ++i) load(i, i);
+  for (int g0 = ga; g0 < gb; g0 += gt) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[h][t][0] = acc[h][t][1] = f64x4{0.0, 0.0, 0.0, 0.0};
+    int s = 0;
+    for (; s + NS < nk; s += NS) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        load(s + i + NS - 1, (i + NS - 1) % NS);
+        step(i);
+      }
+    }
+    // the last one to NS steps (NS - 1 of them requested); k past N add nothing
+    if (s + NS - 1 < nk) load(s + NS - 1, NS - 1);
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      if (s + i < nk) {
+        if (4 * (s + i) + kh >= N) B[i] = double2{0.0, 0.0};
+        step(i);
+      }
+    // the next tile's first steps are in flight during the pair sums
+    rows(g0 + gt);
+#pragma unroll
+    for (int i = 0; i + 1 < NS; ++i) load(i, i);
+    if (busy) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          if (h == 1 && t == 1 && !two1) continue;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int d = kh + 4 * r, row = h == 0 ? 2 * d + t : 32 + (two1 ? 2 * d + t : d);
+            *reinterpret_cast<double2*>(lds + row * X64_LDF + 2 * (16 * wave + cl)) =
+                double2{acc[h][t][0][r], acc[h][t][1][r]};
+          }
+        }
+    }
+    __syncthreads();
+    if (pg < gt && g0 + pg < gb) {
+      const double* F = lds + pg * n * X64_LDF + pw * 2 * n;
+      int p = lt / (n + 1), t = lt - p * (n + 1);
+      while (p < np) {
+        const bool first = t < n - p;
+        const int i = first ? p : n - 1 - p, j = first ? p + t : t - 1;   // second row: j = i + t - (n - p)
+        if (first || 2 * p != n - 1) {
+          const double2 x = *reinterpret_cast<const double2*>(F + i * X64_LDF + 2 * j);
+          const double2 y = *reinterpret_cast<const double2*>(F + j * X64_LDF + 2 * i);
+          const double m = i == j ? 1.0 : 2.0;
+          accr += m * (x.x * y.x - x.y * y.y);
+          acci += m * (x.x * y.y + x.y * y.x);
+        }
+        p += sp;
+        t += stt;
+        if (t > n) { t -= n + 1; ++p; }
+      }
+    }
+    __syncthreads();
+  }
+  // sums of the thread groups (a tree over the group), then of a walker's vectors in order
+  lds[2 * tid] = accr;
+  lds[2 * tid + 1] = acci;
+  int off = 1;
+  while (2 * off < tpb) off *= 2;
+  for (; off > 0; off >>= 1) {
+    __syncthreads();
+    if (lt < off && lt + off < tpb) {
+      lds[2 * tid] += lds[2 * (tid + off)];
+      lds[2 * tid + 1] += lds[2 * (tid + off) + 1];
+    }
+  }
+  __syncthreads();
+  if (tid < gt && w0 + tid < nw) {
+    double xr = 0.0, xi = 0.0;
+    for (int g = 0; g < gt; ++g) {
+      xr += lds[2 * (g * gt + tid) * tpb];
+      xi += lds[2 * (g * gt + tid) * tpb + 1];
+    }
+    const int w = sel ? sel[w0 + tid] : w0 + tid;
+    double* o = Xp + 2 * (((int64_t)tl.z * W + w) * ngt_cap);
+    const int t0 = tl.x * spc, t1 = min((GE + gslot - 1) / gslot, t0 + spc);
+    for (int t = t0; t < t1; ++t) {
+      o[2 * t] = t == t0 ? xr : 0.0;
+      o[2 * t + 1] = t == t0 ? xi : 0.0;
+    }
+  }
+}
+template <bool EVEN>
+struct F_k_exchange64 {
+  static constexpr int NT = X64_NT, OCC = 2;
+  static constexpr bool HAS_OCC = true;
+  template <class... A>
+  __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
+    k_exchange64_body<EVEN>(b, g, a...);
+  }
+};
+template <bool EVEN>
+__global__ __launch_bounds__(X64_NT, 2) void k_exchange64(const double* R, const double* theta, const int* sel,
+                                                          const int* nsel_dev, double* Xp, int N, int GE, int nw, int W,
+                                                          int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
+                                                          int gridx, int gridy, int gridz) {
+  k_exchange64_body<EVEN>(blockIdx3(), gridDim3(), R, theta, sel, nsel_dev, Xp, N, GE, nw, W, Ktot, s0, s1, ngt_cap, gslot,
+                          spc, gridx, gridy, gridz);
+}
+
+// slots a and b (b of a's size; nz = 1: a alone), partials at xp
+void launch_exchange64(const DevState& s, const int* sel, int nsel, const int* nsel_dev, double* xp, Slot a, Slot b, int nz,
+                       hipStream_t st) {
+  // chunks of the vectors: at least 8 where there are as many partials, so that the resident
+  // workgroups of an XCD (8 walker tiles x 8 chunks, tile_id_at) keep their theta in its L2
+  // while R streams; among those the fewest rounds of the 512 resident workgroups
+  const int gslot = exchange_tile_g(a.n), gt = 64 / a.n, ngt = (int)cdivu(s.GE, gslot), gy = (int)cdivu(nsel, gt);
+  int spc = ngt;
+  int64_t best = INT64_MAX;
+  for (int nc = std::min(8, ngt); nc <= std::min(64, ngt); ++nc) {
+    const int per = (int)cdivu(ngt, nc), z = (int)cdivu(ngt, per);
+    const int64_t cost = (int64_t)cdivu((int64_t)z * gy * nz, 512) * (2 * (int64_t)cdivu((int64_t)per * gslot, gt) + 1);
+    if (cost < best) {
+      best = cost;
+      spc = per;
+    }
+  }
+  const int nx = (int)cdivu(ngt, spc);
+#define AFQ_X64(EVEN_)                                                                                                \
+  afq::glaunch<F_k_exchange64<EVEN_>>((k_exchange64<EVEN_>), dim3((unsigned)(nx * gy * nz)), dim3(X64_NT), 0, st, s.R, s.theta, \
+                                      sel, nsel_dev, xp, s.N, s.GE, nsel, s.W, s.Ktot, a, b, s.ngt_cap, gslot, spc, nx, gy, nz)
+  if (a.n % 2 == 0) AFQ_X64(true);
+  else AFQ_X64(false);
+#undef AFQ_X64
+}
+
+}  // namespace afq

@@ -167,8 +167,8 @@ struct DevState {
   // a chunk of R streams through each XCD's L2 once per wave of resident workgroups
   // (0: by shape)
   int xc_chunks = 0;
-  // FP64 exchange kernel: 0 by shape (k_exchange2 with 8 waves), 1 k_exchange (element
-  // loaders), 2 k_exchange2 with 4 waves
+  // FP64 exchange kernel: 0 by shape (k_exchange64 from 4 electrons a slot up, else
+  // k_exchange2), 1 k_exchange (element loaders), 2 k_exchange2
   int xc64_variant = 0;
   // split-BF16 force bias: one workgroup per slot and FP64 combine (true, default), or
   // both slots in one workgroup
@@ -264,6 +264,11 @@ void launch_qr(const DevState& s, hipStream_t st);
 // nsel_dev (nullable): the selection's length on the device; nsel is then the bound the
 // grid is sized for
 void launch_exchange(const DevState& s, const int* sel, int nsel, hipStream_t st, const int* nsel_dev = nullptr);
+// the FP64 exchange kernel for slots of at least X64_NMIN electrons (afq_exchange64.hip):
+// slots a and b (b of a's size; nz = 1: a alone), partials at xp
+constexpr int X64_NMIN = 4;   // its tile holds (64 / n)^2 (vector, walker) pairs, one thread each at least
+void launch_exchange64(const DevState& s, const int* sel, int nsel, const int* nsel_dev, double* xp, Slot a, Slot b, int nz,
+                       hipStream_t st);
 void launch_energy(const DevState& s, const int* sel, int nsel, double delta, hipStream_t st);
 void launch_comb(DevState& s, double zeta, hipStream_t st);
 void launch_live_list(const DevState& s, hipStream_t st);   // s.live / s.nlive: walkers of nonzero weight

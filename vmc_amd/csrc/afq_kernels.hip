@@ -2374,7 +2374,7 @@ __global__ __launch_bounds__(256, 2) void k_exchange(const double* R, const doub
 }
 
 // k_exchange on the pointer-loader engine (MmaF64P: double-buffered stages, no index
-// arithmetic per element): 128 x 128 tiles over 4 (WN = 2) or 8 (WN = 4) waves.
+// arithmetic per element): 128 x 128 tiles over 4 waves (WN = 2).
 template <int WN>
 __device__ __forceinline__ void k_exchange2_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* theta, const int* sel,
                                                           const int* nsel_dev, double* Xp, int N, int GE, int nw,
@@ -2443,40 +2443,29 @@ __global__ __launch_bounds__(128 * WN, 2) void k_exchange2(const double* R, cons
 }
 
 void launch_exchange(const DevState& s, const int* sel, int nsel, hipStream_t st, const int* nsel_dev) {
-  const int n = s.slot[0].n;  // both slots launched in one grid need the same tile shape
-  if (s.nslots == 1 || s.slot[1].n == n) {
-    const int gt = exchange_tile_g(n), wt = exchange_tile_w(n);
-    const int ngt = (int)cdivu(s.GE, gt);
-    const int gy = (int)cdivu(nsel, wt);
-    const dim3 grid(ngt * gy * s.nslots);
-    const Slot b = s.slot[s.nslots > 1 ? 1 : 0];
-    if (s.xc64_variant == 1)
-      afq::glaunch<F_k_exchange>(k_exchange, grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, s.Xp, s.N,
-                         s.GE, nsel, s.W, s.Ktot, s.slot[0], b, s.ngt_cap, ngt, gy, s.nslots);
-    else if (s.xc64_variant == 2)
-      afq::glaunch<F_k_exchange2<2>>(k_exchange2<2>, grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, s.Xp, s.N, s.GE, nsel,
-                         s.W, s.Ktot, s.slot[0], b, s.ngt_cap, ngt, gy, s.nslots);
-    else   // default: the 8-wave pointer-engine kernel
-      afq::glaunch<F_k_exchange2<4>>(k_exchange2<4>, grid, dim3(512), 0, st, s.R, s.theta, sel, nsel_dev, s.Xp, s.N, s.GE, nsel,
-                         s.W, s.Ktot, s.slot[0], b, s.ngt_cap, ngt, gy, s.nslots);
-  } else {
-    for (int z = 0; z < s.nslots; ++z) {
-      const int nz = s.slot[z].n;
-      const int gt = exchange_tile_g(nz), wt = exchange_tile_w(nz);
-      const int ngt = (int)cdivu(s.GE, gt);
-      // a one-slot grid whose z index is the slot: pass the slot as s0 and offset Xp
-      const int gy = (int)cdivu(nsel, wt);
-      double* xp = s.Xp + 2 * (int64_t)z * s.W * s.ngt_cap;
-      if (s.xc64_variant == 1)
-        afq::glaunch<F_k_exchange>(k_exchange, dim3(ngt * gy), dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N,
-                           s.GE, nsel, s.W, s.Ktot, s.slot[z], s.slot[z], s.ngt_cap, ngt, gy, 1);
-      else if (s.xc64_variant == 2)
-        afq::glaunch<F_k_exchange2<2>>(k_exchange2<2>, dim3(ngt * gy), dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N,
-                           s.GE, nsel, s.W, s.Ktot, s.slot[z], s.slot[z], s.ngt_cap, ngt, gy, 1);
-      else
-        afq::glaunch<F_k_exchange2<4>>(k_exchange2<4>, dim3(ngt * gy), dim3(512), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N,
-                           s.GE, nsel, s.W, s.Ktot, s.slot[z], s.slot[z], s.ngt_cap, ngt, gy, 1);
+  // the slots [z0, z0 + nz) in one grid (slots of one size share a tile shape)
+  auto go = [&](int z0, int nz) {
+    const Slot a = s.slot[z0], b = s.slot[z0 + nz - 1];
+    double* xp = s.Xp + 2 * (int64_t)z0 * s.W * s.ngt_cap;
+    if (s.xc64_variant == 0 && a.n >= X64_NMIN) {
+      launch_exchange64(s, sel, nsel, nsel_dev, xp, a, b, nz, st);
+      return;
     }
+    const int gt = exchange_tile_g(a.n), wt = exchange_tile_w(a.n);
+    const int ngt = (int)cdivu(s.GE, gt), gy = (int)cdivu(nsel, wt);
+    const dim3 grid(ngt * gy * nz);
+    if (s.xc64_variant == 1)
+      afq::glaunch<F_k_exchange>(k_exchange, grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel, s.W,
+                                 s.Ktot, a, b, s.ngt_cap, ngt, gy, nz);
+    else
+      afq::glaunch<F_k_exchange2<2>>((k_exchange2<2>), grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel,
+                                     s.W, s.Ktot, a, b, s.ngt_cap, ngt, gy, nz);
+  };
+  if (s.nslots == 1 || s.slot[1].n == s.slot[0].n) {
+    go(0, s.nslots);
+  } else {
+    go(0, 1);
+    go(1, 1);
   }
 }
 
