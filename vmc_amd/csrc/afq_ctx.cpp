@@ -480,7 +480,7 @@ void risk_split_dev(afq_ctx* c) {
 
 void free_mlp(afq_ctx* c) {
   afq::Mlp& m = c->mlp;
-  std::vector<void*> ptrs = {m.mu, m.sd, m.lossbuf, m.X, m.Y, c->cvX};
+  std::vector<void*> ptrs = {m.mu, m.sd, m.lossbuf, m.ws, m.xn, m.X, m.Y, c->cvX};
   for (int l = 0; l < 4; ++l)
     for (void* p : {(void*)m.w[l], (void*)m.b[l], (void*)m.mw[l], (void*)m.vw[l], (void*)m.mb[l], (void*)m.vb[l],
                     (void*)m.gw[l], (void*)m.gb[l], (void*)m.z[l], (void*)m.h[l], (void*)m.dh[l]})
@@ -1257,6 +1257,8 @@ int afq_surrogate_init(afq_ctx* c, int32_t hidden, uint64_t seed, int64_t capaci
   hip_check(scopy(c, m.mu, z0.data(), F * 4, hipMemcpyHostToDevice), "H2D");
   hip_check(scopy(c, m.sd, o1.data(), F * 4, hipMemcpyHostToDevice), "H2D");
   m.lossbuf = dalloc<float>(1);
+  m.xn = dalloc<float>((int64_t)m.Bcap * F);
+  m.ws = dalloc<float>(afq::mlp_ws_floats(m.dims, m.Bcap));
   m.cap = capacity;
   if (capacity > 0) {
     m.X = dalloc<float>(capacity * F);
@@ -1419,7 +1421,7 @@ int afq_surrogate_train(afq_ctx* c, int32_t epochs, int32_t batch, double lr, ui
       for (int64_t b0 = 0; b0 + batch <= ntr; b0 += batch) {
         afq::mlp_forward(m, m.X, didx + b0, batch, c->stream);
         afq::mlp_loss(m, m.Y, didx + b0, batch, c->stream);
-        afq::mlp_backward(m, m.X, didx + b0, batch, c->stream);
+        afq::mlp_backward(m, batch, c->stream);
         afq::mlp_adam(m, (float)lr, c->stream);
       }
       launch_check("train");
@@ -1514,7 +1516,7 @@ int afq_surrogate_grad(afq_ctx* c, const float* X, const float* t, int32_t B, fl
   hip_check(scopy(c, dT, t, (size_t)B * 4, hipMemcpyHostToDevice), "H2D");
   afq::mlp_forward(m, dX, nullptr, B, c->stream);
   const float l = afq::mlp_loss(m, dT, nullptr, B, c->stream);
-  afq::mlp_backward(m, dX, nullptr, B, c->stream);
+  afq::mlp_backward(m, B, c->stream);
   launch_check("grad");
   int64_t off = 0;
   for (int l2 = 0; l2 < 4; ++l2) {

@@ -555,9 +555,11 @@ struct MmaBF16 {
 // ---------------------------------------------------------------------------
 // BF16 engine with element loaders: la(r, k) and lb(k, c) return floats that
 // are rounded to bf16 when staged in LDS (the MLP's GEMMs, where operands come
-// from FP32 master weights / activations in several layouts).
+// from FP32 master weights / activations in several layouts; the next stage's loads are in
+// flight during this one's MFMAs, so the rounding waits for the write to LDS).  A_ROWFAST: consecutive
+// threads load consecutive rows of A at one k (an operand that lies transposed in memory).
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int WAVES_M, int WAVES_N>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool A_ROWFAST = false>
 struct MmaBF16E {
   static constexpr int BK = 32;
   static constexpr int LDK = BK + 8;
@@ -584,17 +586,17 @@ struct MmaBF16E {
     u16* As = reinterpret_cast<u16*>(ldsv);
     u16* Bs = As + BM * LDK;
     const int tid = threadIdx.x;
-    u16 ra[A_PER_T], rb[B_PER_T];
+    float ra[A_PER_T], rb[B_PER_T];
     auto fetch = [&](int k0) {
 #pragma unroll
       for (int q = 0; q < A_PER_T; ++q) {
-        const int e = tid + q * NT, r = e / BK, kk = e % BK;
-        ra[q] = f2bf_bits(la(r, k0 + kk));
+        const int e = tid + q * NT, r = A_ROWFAST ? e % BM : e / BK, kk = A_ROWFAST ? e / BM : e % BK;
+        ra[q] = la(r, k0 + kk);
       }
 #pragma unroll
       for (int q = 0; q < B_PER_T; ++q) {
         const int e = tid + q * NT, kk = e / BN, c = e % BN;
-        rb[q] = f2bf_bits(lb(k0 + kk, c));
+        rb[q] = lb(k0 + kk, c);
       }
     };
     const int nst = (K + BK - 1) / BK;
@@ -602,13 +604,13 @@ struct MmaBF16E {
     for (int s = 0; s < nst; ++s) {
 #pragma unroll
       for (int q = 0; q < A_PER_T; ++q) {
-        const int e = tid + q * NT, r = e / BK, kk = e % BK;
-        As[r * LDK + kk] = ra[q];
+        const int e = tid + q * NT, r = A_ROWFAST ? e % BM : e / BK, kk = A_ROWFAST ? e / BM : e % BK;
+        As[r * LDK + kk] = f2bf_bits(ra[q]);
       }
 #pragma unroll
       for (int q = 0; q < B_PER_T; ++q) {
         const int e = tid + q * NT, kk = e / BN, c = e % BN;
-        Bs[c * LDK + kk] = rb[q];
+        Bs[c * LDK + kk] = f2bf_bits(rb[q]);
       }
       __syncthreads();
       if (s + 1 < nst) fetch((s + 1) * BK);

@@ -201,6 +201,8 @@ struct Mlp {
   float* mu = nullptr; float* sd = nullptr;
   float t_mu = 0.f, t_sd = 1.f;
   float* lossbuf = nullptr;
+  float* xn = nullptr;   // standardised input rows of the batch, Bcap x F
+  float* ws = nullptr;   // partial weight gradients of a batch's chunks (mlp_ws_floats for Bcap rows)
   int Bcap = 0;
   int t = 0;
   double calib_b = 1.0;                     // calibration slope of the last training
@@ -208,8 +210,9 @@ struct Mlp {
   int64_t n = 0, cap = 0;
   bool ready = false;
 };
+int64_t mlp_ws_floats(const int* dims, int B);   // workspace of mlp_backward for batches of at most B rows
 void mlp_forward(const Mlp& m, const float* X, const int* idx, int B, hipStream_t st);
-void mlp_backward(const Mlp& m, const float* X, const int* idx, int B, hipStream_t st);
+void mlp_backward(const Mlp& m, int B, hipStream_t st);
 float mlp_loss(const Mlp& m, const float* t, const int* idx, int B, hipStream_t st);
 void mlp_adam(Mlp& m, float lr, hipStream_t st);
 void launch_features(const DevState& s, const int* idx, int n, float* X, int64_t dst0, hipStream_t st);
