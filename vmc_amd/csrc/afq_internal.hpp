@@ -261,6 +261,23 @@ void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st);  // s
 void launch_green(const DevState& s, bool all_walkers, hipStream_t st);
 void launch_green_pre(const DevState& s, bool all_walkers, hipStream_t st);   // S, S^-1, log det S
 void launch_theta_post(const DevState& s, hipStream_t st);                   // theta, e1 of the live walkers
+// arguments of the Green's function kernels
+struct GreenArgs {
+  const double* psi; double* theta; double* logdet; double* e1; const double* weights; double* Sg;
+  // fresh[w] = 1 when k_invert took walker w (its S^-1 in Sg is current); with
+  // post = 1, k_theta takes the fresh walkers of nonzero weight only
+  int* fresh = nullptr; int post = 0;
+  // with tbh != nullptr, k_theta also writes theta split into Tb (hi tbh, lo tbl),
+  // laid out as k_theta_split writes it
+  unsigned short* tbh = nullptr; unsigned short* tbl = nullptr; int Np = 0, ctot = 0;
+  const double* phi0; const double* phi1; const double* hphi0; const double* hphi1;
+  int64_t ms, Ktot; int64_t det_off0, det_off1; int N, nslots, W; Slot s0, s1; int all;
+};
+constexpr int GN_MAX = 64;                              // electrons per slot at most
+constexpr int SG_LD = 2 * GN_MAX;                       // doubles per row of an Sg matrix
+constexpr int64_t SG_MAT = (int64_t)GN_MAX * SG_LD;     // doubles per (walker, slot)
+void launch_overlap(const GreenArgs& a, hipStream_t st);   // afq_green.hip
+void launch_theta(const GreenArgs& a, hipStream_t st);
 void launch_weight(const DevState& s, double eshift, bool update_weights, hipStream_t st);
 void launch_logO_from_logdet(const DevState& s, hipStream_t st);
 void launch_qr(const DevState& s, hipStream_t st);

@@ -1371,63 +1371,16 @@ void launch_propagate(const DevState& s, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ Green's function
-constexpr int GN_MAX = 64;
-
-// The Green's function in three batched kernels:
+// The Green's function in three batched kernels (1 and 3 in afq_green.hip):
 //  1. k_overlap: S = Phi_s^T psi for every walker of a slot as one GEMM over the
 //     W * 2n real columns (FP64 MFMA), into Sg[w][slot] (64 x 128 doubles each);
 //  2. k_invert: S^-1 and log det S per (walker, slot) by Gauss-Jordan elimination with
 //     partial pivoting, the matrix held in registers (lane = row, wave q = complex
 //     columns CPW q .. CPW q + CPW - 1), so a workgroup needs only 3 KB of LDS;
-//  3. k_theta_r: theta = psi S^-1 (FP64 MFMA, S^-1 held in registers) and the one-body
+//  3. k_theta: theta = psi S^-1 (FP64 MFMA, S^-1 held in LDS) and the one-body
 //     partial e1 = sum theta o (h1 Phi).
 // In a propagation step 1-2 run before the weight update (the overlap ratio needs
 // log det S of every propagated walker) and 3 after it, for the walkers still alive.
-struct GreenArgs {
-  const double* psi; double* theta; double* logdet; double* e1; const double* weights; double* Sg;
-  // fresh[w] = 1 when k_invert took walker w (its S^-1 in Sg is current); with
-  // post = 1, k_theta_r takes the fresh walkers of nonzero weight only
-  int* fresh = nullptr; int post = 0;
-  // with tbh != nullptr, k_theta_r also writes theta split into Tb (hi tbh, lo tbl),
-  // laid out as k_theta_split writes it
-  u16* tbh = nullptr; u16* tbl = nullptr; int Np = 0, ctot = 0;
-  const double* phi0; const double* phi1; const double* hphi0; const double* hphi1;
-  int64_t ms, Ktot; int64_t det_off0, det_off1; int N, nslots, W; Slot s0, s1; int all;
-};
-constexpr int SG_LD = 2 * GN_MAX;                       // doubles per row of an Sg matrix
-constexpr int64_t SG_MAT = (int64_t)GN_MAX * SG_LD;     // doubles per (walker, slot)
-
-__device__ __forceinline__ void k_overlap_body(const uint3 bid_, const uint3 gdim_, GreenArgs a, int si, int gridx) {
-  using ES = MmaF64<64, 128, 2, 2, true, true>;
-  __shared__ double stage[ES::LDS_DOUBLES];
-  const Slot sl = si == 0 ? a.s0 : a.s1;
-  const int n = sl.n, n2 = 2 * n, ncol = a.W * n2;
-  const int q0 = bid_.x * 128;
-  const double* phi = sl.phi == 0 ? a.phi0 : a.phi1;
-  const int64_t doff = 2 * (sl.det == 0 ? a.det_off0 : a.det_off1);
-  ES e;
-  e.run([&](int r, int k) { return (r < n && k < a.N) ? phi[(int64_t)k * n + r] : 0.0; },
-        DetColsB{a.psi, 2 * a.ms, doff, a.N, n2, q0, ncol}, a.N, stage);
-  e.store([&](int r, int c, double v) {
-    const int q = q0 + c;
-    if (r >= n || q >= ncol) return;
-    const int w = q / n2, cc = q - w * n2;
-    if (!a.all && a.weights[w] <= 1e-8) return;
-    a.Sg[((int64_t)w * a.nslots + si) * SG_MAT + (int64_t)r * SG_LD + cc] = v;
-  });
-}
-struct F_k_overlap {
-  static constexpr int NT = 256, OCC = 3;
-  static constexpr bool HAS_OCC = true;
-  template <class... A>
-  __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_overlap_body(b, g, a...);
-  }
-};
-__global__ __launch_bounds__(256, 3) void k_overlap(GreenArgs a, int si, int gridx) {
-  k_overlap_body(blockIdx3(), gridDim3(), a, si, gridx);
-}
-
 __device__ __forceinline__ double readlane_f64(double x, int l) {
   const long long b = __double_as_longlong(x);
   const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
@@ -1562,7 +1515,7 @@ __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim
 }
 template <int CPW>
 struct F_k_invert {
-  static constexpr int NT = 64 * (64 / CPW), OCC = CPW == 16 ? 3 : 2;
+  static constexpr int NT = 256, OCC = CPW == 16 ? 3 : 4;
   static constexpr bool HAS_OCC = true;
   template <class... A>
   __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
@@ -1570,149 +1523,22 @@ struct F_k_invert {
   }
 };
 template <int CPW>
-__global__ __launch_bounds__(64 * (64 / CPW), CPW == 16 ? 3 : 2) void k_invert(GreenArgs a) {
+__global__ __launch_bounds__(256, CPW == 16 ? 3 : 4) void k_invert(GreenArgs a) {
   k_invert_body<CPW>(blockIdx3(), gridDim3(), a);
 }
 
-// theta = psi S^-1 with S^-1 held in registers: the real embedding B = [[S_re, S_im],
-// [-S_im, S_re]] of S^-1 (2n x 2n, zero-padded to 128 x 128) is split by columns over
-// eight waves (wave v: columns 16v .. 16v+15, as MFMA B fragments, 32 doubles a lane),
-// and the rows of psi stream through LDS 16 at a time (double-buffered, fetched into
-// registers one tile ahead, one barrier per row tile), so each row tile is 32 FP64 MFMA
-// K steps per wave with no other traffic.  Also the one-body partial
-// e1 = sum theta o (h1 Phi).
-constexpr int TR_KS = 2 * GN_MAX / 4;   // K steps of 4
-constexpr int TR_LDA = 20;              // LDS row pitch of a staged A tile [k][16 rows] (doubles)
-constexpr int TR_NT = 512;
-__device__ __forceinline__ void k_theta_r_body(const uint3 bid_, const uint3 gdim_, GreenArgs a) {
-  __shared__ double As[2][2 * GN_MAX * TR_LDA];
-  __shared__ double red[16];
-  const int w = bid_.x, si = bid_.y;
-  if (a.post ? (!a.fresh[w] || a.weights[w] == 0.0) : (!a.all && a.weights[w] <= 1e-8)) return;
-  const Slot sl = si == 0 ? a.s0 : a.s1;
-  const int n = sl.n, N = a.N, n2 = 2 * n;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const double* psi = a.psi + (int64_t)w * 2 * a.ms + 2 * (sl.det == 0 ? a.det_off0 : a.det_off1);
-  const double* hphi = sl.phi == 0 ? a.hphi0 : a.hphi1;
-  const double* Si = a.Sg + ((int64_t)w * a.nslots + si) * SG_MAT;
-  double* th = a.theta + (int64_t)w * 2 * a.Ktot + 2 * sl.koff;
-  const int c = 16 * wave + (lane & 15);   // this lane's output column
-  // B fragments: lane holds B[k = 4 ks + (lane >> 4)][c]
-  double b[TR_KS];
-#pragma unroll
-  for (int ks = 0; ks < TR_KS; ++ks) {
-    const int k = 4 * ks + (lane >> 4);
-    double v = 0.0;
-    if (k < n2 && c < n2) {
-      const int j = c >> 1, comp = c & 1;
-      if (k < n) v = Si[k * SG_LD + 2 * j + comp];
-      else v = comp ? Si[(k - n) * SG_LD + 2 * j] : -Si[(k - n) * SG_LD + 2 * j + 1];
-    }
-    b[ks] = v;
-  }
-  // A tile: psi rows r0 .. r0+15 as [k][row], k < n the real and k >= n the imaginary
-  // parts; k >= 2n stays zero
-  const int ntile = (N + 15) >> 4;
-  for (int e = tid; e < 2 * 2 * GN_MAX * TR_LDA; e += TR_NT) (&As[0][0])[e] = 0.0;
-  __syncthreads();
-  // a tile's elements e = tid + 512 i (at most 16 x 128 = 4 a thread): fetched into
-  // registers one tile ahead, written to LDS after this tile's MFMAs; the element ->
-  // (global offset within the tile, LDS offset) map is the same for every tile
-  int goff[4], loff[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int e = tid + TR_NT * i, r = e / n2, q = e - r * n2;
-    const int k = (q & 1) ? n + (q >> 1) : (q >> 1);
-    goff[i] = e < 16 * n2 ? e : -1;   // = r n2 + q
-    loff[i] = k * TR_LDA + r;
-  }
-  double ra[4];
-  // (loads without a branch: an element outside the tile reads the tile's first one and
-  // is replaced by zero, so that no wait for the prefetch lands before the MFMAs)
-  auto fetch = [&](int r0) {
-    const int lim = (N - r0) * n2;   // elements of the tile's rows below N
-    const double* base = psi + (int64_t)r0 * n2;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bool ok = goff[i] >= 0 && goff[i] < lim;
-      const double v = base[ok ? goff[i] : 0];
-      ra[i] = ok ? v : 0.0;
-    }
-  };
-  auto put = [&](double* dstA) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (goff[i] >= 0) dstA[loff[i]] = ra[i];
-  };
-  double e1re = 0.0, e1im = 0.0;
-  fetch(0);
-  put(As[0]);
-  __syncthreads();
-  for (int rt = 0; rt < ntile; ++rt) {
-    const double* A = As[rt & 1];
-    // the tile's A operands read from LDS first (the reads in flight together, not one
-    // pair per two MFMAs), then the global loads of the next tile (the last tile again at
-    // the end, not stored) and of h1 Phi, then two accumulator chains over the even and
-    // the odd K steps, so that a wave has two independent MFMAs to issue; the scheduling
-    // barriers keep that order (else each read sinks to its MFMA)
-    double av[TR_KS];
-#pragma unroll
-    for (int ks = 0; ks < TR_KS; ++ks) av[ks] = A[(4 * ks + (lane >> 4)) * TR_LDA + (lane & 15)];
-    __builtin_amdgcn_sched_barrier(0);
-    fetch(16 * min(rt + 1, ntile - 1));
-    double hv[4];   // h1 Phi at this tile's output positions, for e1
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = 16 * rt + (lane >> 4) + 4 * r;
-      const bool ok = rr < N && c < n2;
-      const double v = hphi[ok ? (int64_t)rr * n + (c >> 1) : 0];
-      hv[r] = ok ? v : 0.0;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0}, acc2 = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int ks = 0; ks < TR_KS; ks += 2) {
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ks], b[ks], acc, 0, 0, 0);
-      acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ks + 1], b[ks + 1], acc2, 0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] += acc2[r];
-    if (rt + 1 < ntile) put(As[(rt + 1) & 1]);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = 16 * rt + (lane >> 4) + 4 * r;
-      if (rr < N && c < n2) {
-        th[(int64_t)rr * n2 + c] = acc[r];
-        if (c & 1) e1im += acc[r] * hv[r]; else e1re += acc[r] * hv[r];
-      }
-      // the split copy, pad rows N .. Np-1 included (psi's rows past N load as zero)
-      if (a.tbh && rr < a.Np && c < n2) {
-        u16 h, l;
-        split_bf16(acc[r], h, l);
-        const int64_t ta = (((int64_t)w * 2 + (c & 1)) * (a.ctot / 2) + (si == 0 ? 0 : a.s0.n) + (c >> 1)) * a.Np + rr;
-        a.tbh[ta] = h;
-        a.tbl[ta] = l;
-      }
-    }
-    __syncthreads();
-  }
-  e1re = block_sum(e1re, red);
-  e1im = block_sum(e1im, red);
-  if (tid == 0) {
-    a.e1[2 * ((int64_t)w * a.nslots + si)] = e1re;
-    a.e1[2 * ((int64_t)w * a.nslots + si) + 1] = e1im;
-  }
-}
-struct F_k_theta_r {
-  static constexpr int NT = TR_NT, OCC = 2;
-  static constexpr bool HAS_OCC = true;
-  template <class... A>
-  __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_theta_r_body(b, g, a...);
-  }
-};
-__global__ __launch_bounds__(TR_NT, 2) void k_theta_r(GreenArgs a) {
-  k_theta_r_body(blockIdx3(), gridDim3(), a);
+// CPW columns a wave and as many waves as the slots' columns fill: a wave's work per step is
+// its columns whether they hold data or not (2048 matrices of n = 20: 59 us as three waves of
+// 8 columns, 99 as four of 16)
+static void launch_invert(const GreenArgs& a, hipStream_t st) {
+  const int nmax = std::max(a.s0.n, a.nslots > 1 ? a.s1.n : 0);
+  const dim3 grid(a.W, a.nslots);
+  if (nmax <= 16)
+    afq::glaunch<F_k_invert<4>>(k_invert<4>, grid, dim3(64 * cdivu(nmax, 4)), 0, st, a);
+  else if (nmax <= 32)
+    afq::glaunch<F_k_invert<8>>(k_invert<8>, grid, dim3(64 * cdivu(nmax, 8)), 0, st, a);
+  else
+    afq::glaunch<F_k_invert<16>>(k_invert<16>, grid, dim3(64 * cdivu(nmax, 16)), 0, st, a);   // 4 waves: faster than 8 at n = 60
 }
 
 static GreenArgs green_args(const DevState& s, bool all) {
@@ -1730,11 +1556,8 @@ void launch_green_pre(const DevState& s, bool all, hipStream_t st) {
   s.tb_post = false;
   GreenArgs a = green_args(s, all);
   a.fresh = s.gfresh;
-  for (int si = 0; si < s.nslots; ++si) {
-    const int gx = (int)cdivu((int64_t)s.W * 2 * s.slot[si].n, 128);
-    afq::glaunch<F_k_overlap>(k_overlap, dim3(gx), dim3(256), 0, st, a, si, gx);
-  }
-  afq::glaunch<F_k_invert<16>>(k_invert<16>, dim3(s.W, s.nslots), dim3(256), 0, st, a);   // 4 waves: faster than 8 at n = 60
+  launch_overlap(a, st);
+  launch_invert(a, st);
 }
 // theta = psi S^-1 (and e1) after the weight update, for the walkers launch_green_pre
 // took that are still alive: the others are never read before the next step recomputes
@@ -1751,19 +1574,16 @@ void launch_theta_post(const DevState& s, hipStream_t st) {
     a.Np = s.Np;
     a.ctot = s.ctot;
   }
-  afq::glaunch<F_k_theta_r>(k_theta_r, dim3(s.W, s.nslots), dim3(TR_NT), 0, st, a);
+  launch_theta(a, st);
   s.tb_post = a.tbh != nullptr;
 }
 void launch_green(const DevState& s, bool all, hipStream_t st) {
   s.tb_live = false;
   s.tb_post = false;
   const GreenArgs a = green_args(s, all);
-  for (int si = 0; si < s.nslots; ++si) {
-    const int gx = (int)cdivu((int64_t)s.W * 2 * s.slot[si].n, 128);
-    afq::glaunch<F_k_overlap>(k_overlap, dim3(gx), dim3(256), 0, st, a, si, gx);
-  }
-  afq::glaunch<F_k_invert<16>>(k_invert<16>, dim3(s.W, s.nslots), dim3(256), 0, st, a);   // 4 waves: faster than 8 at n = 60
-  afq::glaunch<F_k_theta_r>(k_theta_r, dim3(s.W, s.nslots), dim3(TR_NT), 0, st, a);
+  launch_overlap(a, st);
+  launch_invert(a, st);
+  launch_theta(a, st);
 }
 
 // ------------------------------------------------------------------ weights
@@ -2570,7 +2390,7 @@ __device__ __forceinline__ void k_theta_split_body(const uint3 bid_, const uint3
   __shared__ double tile[32 * 129];
   if (nsel_dev && (int)bid_.x >= *nsel_dev) return;
   const int w = sel ? sel[bid_.x] : bid_.x;
-  if (skip && skip[w]) return;   // split already (by k_theta_r)
+  if (skip && skip[w]) return;   // split already (by k_theta)
   const Slot sl = bid_.y == 0 ? s0 : s1;
   const int n2 = 2 * sl.n;
   const int coff = bid_.y == 0 ? 0 : 2 * s0.n;
@@ -3400,7 +3220,7 @@ __global__ __launch_bounds__(256) void k_fb_combine(const float* __restrict__ pa
 
 void launch_force_bias_lp(const DevState& s, int prec, hipStream_t st) {
   launch_live_list(s, st);
-  // the live walkers k_theta_r split straight after their theta are skipped
+  // the live walkers k_theta split straight after their theta are skipped
   afq::glaunch<F_k_theta_split>(k_theta_split, dim3(s.W, s.nslots), dim3(256), 0, st, s.theta, s.live, s.nlive, s.Tb_hi,
                      s.Tb_lo, s.N, s.Np, s.Ktot, s.slot[0], s.slot[s.nslots > 1 ? 1 : 0], s.ctot,
                      (const int*)(s.tb_post ? s.gfresh : nullptr));
