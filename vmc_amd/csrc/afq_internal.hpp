@@ -281,6 +281,7 @@ void launch_theta(const GreenArgs& a, hipStream_t st);
 void launch_weight(const DevState& s, double eshift, bool update_weights, hipStream_t st);
 void launch_logO_from_logdet(const DevState& s, hipStream_t st);
 void launch_qr(const DevState& s, hipStream_t st);
+bool launch_qr_cols(const DevState& s, hipStream_t st);   // afq_qr.hip; false where it does not apply
 // nsel_dev (nullable): the selection's length on the device; nsel is then the bound the
 // grid is sized for
 void launch_exchange(const DevState& s, const int* sel, int nsel, hipStream_t st, const int* nsel_dev = nullptr);
