@@ -19,7 +19,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libvmc_afqmc.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
-SOURCES = ["afq_kernels.hip", "afq_force_bias.hip", "afq_prop64.hip", "afq_exchange64.hip", "afq_green.hip", "afq_qr.hip", "afq_exchange_pw2.hip", "afq_exchange_pw2x3.hip", "afq_mlp.hip", "afq_ctx.cpp", "afq_driver.cpp",
+SOURCES = ["afq_kernels.hip", "afq_force_bias.hip", "afq_prop64.hip", "afq_exchange64.hip", "afq_green.hip", "afq_qr.hip", "afq_vhs64.hip", "afq_exchange_pw2.hip", "afq_exchange_pw2x3.hip", "afq_mlp.hip", "afq_ctx.cpp", "afq_driver.cpp",
            "afq_noalloc.cpp"]
 # per-file hipcc options: the pair-wise exchange keeps its MFMA accumulators in VGPRs
 SOURCE_FLAGS = {"afq_exchange_pw2.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}

@@ -604,14 +604,14 @@ int afq_create(const afq_ham* ham, const afq_trial* left, const afq_params* para
     // device Hamiltonian / trial
     double* Ld = dalloc<double>((size_t)G * NN);
     upload(Ld, c->chol.data(), (size_t)G * NN, c->stream);
-    s.Lp = dalloc<double>((size_t)G * s.T);
+    s.Lp = dalloc<double>((size_t)G * s.T + 1);   // pairs of columns are read at any offset
     afq::launch_pack_chol(Ld, s.Lp, N, G, s.T, s.ref_compat, c->stream);
     launch_check("pack_chol");
     double* Ldd = nullptr;  // down-spin vectors (unrestricted integrals)
     if (uints) {
       Ldd = dalloc<double>((size_t)G * NN);
       upload(Ldd, c->chold.data(), (size_t)G * NN, c->stream);
-      s.Lp2 = dalloc<double>((size_t)G * s.T);
+      s.Lp2 = dalloc<double>((size_t)G * s.T + 1);
       afq::launch_pack_chol(Ldd, s.Lp2, N, G, s.T, s.ref_compat, c->stream);
       launch_check("pack_chol");
     }

@@ -131,78 +131,6 @@ void launch_fields(const DevState& s, const double* draws, uint64_t seed, uint64
                      s.sft, s.G, s.dt, (int)s.ref_compat, seed, step, s.d_step);
 }
 
-// ------------------------------------------------------------------ VHS
-struct VhsA {  // A((w,c), g) = field[w][g][c]
-  const double* f; int G; int row0, nrow;
-  __device__ double operator()(int r, int k) const {
-    const int q = row0 + r;
-    if (q >= nrow || k >= G) return 0.0;
-    return f[(int64_t)(q >> 1) * 2 * G + 2 * k + (q & 1)];
-  }
-};
-struct VhsB {  // B(g, t) = Lp[g][t]
-  const double* Lp; int64_t T; int G; int64_t t0;
-  __device__ double operator()(int k, int c) const {
-    const int64_t t = t0 + c;
-    if (k >= G || t >= T) return 0.0;
-    return Lp[(int64_t)k * T + t];
-  }
-};
-constexpr int VHS_BM = 128, VHS_BN = 128;
-__device__ __forceinline__ void k_vhs_body(const uint3 bid_, const uint3 gdim_, const double* fields, const double* Lp, double* P,
-                                             const double* weights, int G, int W, int64_t T, int N,
-                                             int ref_compat, int gridx, int gridy) {
-  using Eng = MmaF64<VHS_BM, VHS_BN, 2, 2, false, true>;
-  __shared__ double lds[Eng::LDS_DOUBLES];
-  const TileId tl = tile_id_at(bid_.x, gridx, gridy, 1, 8);
-  const int row0 = tl.y * VHS_BM;
-  const int64_t t0 = (int64_t)tl.x * VHS_BN;
-  // skip tiles whose walkers are all dead
-  bool any = false;
-  for (int q = row0; q < min(row0 + VHS_BM, 2 * W); q += 2) any |= weights[q >> 1] > 1e-8;
-  if (!any) return;
-  Eng e;
-  e.run(VhsA{fields, G, row0, 2 * W}, VhsB{Lp, T, G, t0}, G, lds);
-  e.store([&](int r, int c, double v) {
-    const int q = row0 + r;
-    const int64_t t = t0 + c;
-    if (q >= 2 * W || t >= T) return;
-    // packed t = i(i+1)/2 + j (j <= i) -> both triangles of the N x N matrix
-    int i = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-    if ((int64_t)(i + 1) * (i + 2) / 2 <= t) ++i;
-    if ((int64_t)i * (i + 1) / 2 > t) --i;
-    const int j = (int)(t - (int64_t)i * (i + 1) / 2);
-    const double x = ref_compat ? (double)(float)v : v;
-    double* Pq = P + (int64_t)q * N * N;
-    Pq[(int64_t)i * N + j] = x;
-    Pq[(int64_t)j * N + i] = x;
-  });
-}
-struct F_k_vhs {
-  static constexpr int NT = 256, OCC = 2;
-  static constexpr bool HAS_OCC = true;
-  template <class... A>
-  __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_vhs_body(b, g, a...);
-  }
-};
-__global__ __launch_bounds__(256, 2) void k_vhs(const double* fields, const double* Lp, double* P,
-                                             const double* weights, int G, int W, int64_t T, int N,
-                                             int ref_compat, int gridx, int gridy) {
-  k_vhs_body(blockIdx3(), gridDim3(), fields, Lp, P, weights, G, W, T, N, ref_compat, gridx, gridy);
-}
-
-void launch_vhs(const DevState& s, hipStream_t st) {
-  const int gx = (int)cdivu(s.T, VHS_BN), gy = (int)cdivu(2 * (int64_t)s.W, VHS_BM);
-  afq::glaunch<F_k_vhs>(k_vhs, dim3(gx * gy), dim3(256), 0, st, s.fields, s.Lp, s.P, s.weights, s.G, s.W, s.T,
-                     s.N, (int)s.ref_compat, gx, gy);
-  // unrestricted integrals: the down-spin VHS from the down-spin vectors
-  // (propagatePhaselessU, DQMC/DQMCWalker.cpp:525-530)
-  if (s.uints)
-    afq::glaunch<F_k_vhs>(k_vhs, dim3(gx * gy), dim3(256), 0, st, s.fields, s.Lp2, s.P2, s.weights, s.G, s.W, s.T,
-                       s.N, (int)s.ref_compat, gx, gy);
-}
-
 // ------------------------------------------------------------------ propagation
 // out = E * src for determinant d of every walker (walkers folded into columns).
 struct ExpA {
