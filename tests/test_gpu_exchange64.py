@@ -59,3 +59,11 @@ def test_exchange_matches_numpy(case):
             mag += 0.5 * np.einsum("gij,gji->", a, a)
         assert abs(ek[w] - ref) <= 1e-12 * mag
     assert ek[W // 2] == 0.0
+
+
+@pytest.mark.parametrize("case", [
+    # at most 48 rows and columns: three waves a workgroup
+    (40, 22, 22, 45, 7, 20), (41, 23, 23, 30, 4, 30), (24, 24, 24, 9, 3, 9), (33, 33, 33, 19, 3, 19), (49, 48, 48, 11, 2, 11),
+], ids=lambda c: "N%d_%d_%d_G%d_W%d" % c[:5])
+def test_exchange_three_waves_matches_numpy(case):
+    test_exchange_matches_numpy(case)

@@ -29,16 +29,19 @@ static inline unsigned cdivu(int64_t a, int64_t b) { return (unsigned)((a + b - 
 // operands took 56 and 3.3 ms (two 8-byte LDS reads per MFMA), one with 8-byte global loads
 // per tile 49.2 and 3.06.  NS = 6 against 4: equal at N = 100 and 300, 3% faster on systems of
 // N = 20 to 120.
-constexpr int X64_LDF = 130;   // 16-byte rows; transposed 16-byte reads of 16 lanes on 64 banks
-constexpr int X64_NT = 256;
+template <int WAVES>
+struct X64Shape {
+  static constexpr int NT = 64 * WAVES, ROWS = 16 * WAVES, OCC = WAVES == 4 ? 2 : 3;
+  static constexpr int LDF = 2 * ROWS + 2;   // 16-byte rows; transposed 16-byte reads of 16 lanes on 64 banks
+};
 typedef double __attribute__((ext_vector_type(2), aligned(8))) x64_pair;   // two rows of R, 8-byte aligned
-template <bool EVEN>
+template <bool EVEN, int WAVES>
 __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* theta,
                                                   const int* sel, const int* nsel_dev, double* Xp, int N, int GE, int nw,
                                                   int W, int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
                                                   int gridx, int gridy, int gridz) {
-  constexpr int NS = 6;
-  __shared__ __attribute__((aligned(16))) double lds[64 * X64_LDF];
+  constexpr int NS = 6, NT = X64Shape<WAVES>::NT, LDF = X64Shape<WAVES>::LDF;
+  __shared__ __attribute__((aligned(16))) double lds[X64Shape<WAVES>::ROWS * LDF];
   const TileId tl = tile_id_at(bid_.x, gridx, gridy, gridz, 8);
   const Slot sl = tl.z == 0 ? s0 : s1;
   const int n = sl.n, gt = 64 / n, w0 = tl.y * gt, nrow = gt * n;
@@ -50,7 +53,7 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
   const bool busy = 16 * wave < nrow;   // this wave's columns hold data
   // rows 32 .. nrow (gt n > 32 always): as two tiles, or as one where at most 16 (row 32 + cl)
   const int rest = nrow - 32;
-  const bool two1 = rest > 16;
+  const bool two1 = WAVES == 4 && rest > 16;
   // A: rows past the data read a valid one
   auto split = [&](int r, int& g, int& e) {
     r = min(r, nrow - 1);
@@ -112,7 +115,7 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
     }
   };
   // pair sums: threads [b tpb, (b + 1) tpb) take block b = (vector b / gt, walker b % gt) of a tile
-  const int tpb = X64_NT / (gt * gt);
+  const int tpb = NT / (gt * gt);
   const int blk = tid / tpb, lt = tid - blk * tpb, pg = blk / gt, pw = blk - pg * gt;
   // units (p, t): rows p and n - 1 - p share the n + 1 pairs i <= j
   const int np = (n + 1) >> 1, sp = tpb / (n + 1), stt = tpb - sp * (n + 1);
@@ -154,21 +157,21 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int d = kh + 4 * r, row = h == 0 ? 2 * d + t : 32 + (two1 ? 2 * d + t : d);
-            *reinterpret_cast<double2*>(lds + row * X64_LDF + 2 * (16 * wave + cl)) =
+            *reinterpret_cast<double2*>(lds + row * LDF + 2 * (16 * wave + cl)) =
                 double2{acc[h][t][0][r], acc[h][t][1][r]};
           }
         }
     }
     __syncthreads();
     if (pg < gt && g0 + pg < gb) {
-      const double* F = lds + pg * n * X64_LDF + pw * 2 * n;
+      const double* F = lds + pg * n * LDF + pw * 2 * n;
       int p = lt / (n + 1), t = lt - p * (n + 1);
       while (p < np) {
         const bool first = t < n - p;
         const int i = first ? p : n - 1 - p, j = first ? p + t : t - 1;   // second row: j = i + t - (n - p)
         if (first || 2 * p != n - 1) {
-          const double2 x = *reinterpret_cast<const double2*>(F + i * X64_LDF + 2 * j);
-          const double2 y = *reinterpret_cast<const double2*>(F + j * X64_LDF + 2 * i);
+          const double2 x = *reinterpret_cast<const double2*>(F + i * LDF + 2 * j);
+          const double2 y = *reinterpret_cast<const double2*>(F + j * LDF + 2 * i);
           const double m = i == j ? 1.0 : 2.0;
           accr += m * (x.x * y.x - x.y * y.y);
           acci += m * (x.x * y.y + x.y * y.x);
@@ -208,21 +211,21 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
     }
   }
 }
-template <bool EVEN>
+template <bool EVEN, int WAVES>
 struct F_k_exchange64 {
-  static constexpr int NT = X64_NT, OCC = 2;
+  static constexpr int NT = 64 * WAVES, OCC = WAVES == 4 ? 2 : 3;
   static constexpr bool HAS_OCC = true;
   template <class... A>
   __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_exchange64_body<EVEN>(b, g, a...);
+    k_exchange64_body<EVEN, WAVES>(b, g, a...);
   }
 };
-template <bool EVEN>
-__global__ __launch_bounds__(X64_NT, 2) void k_exchange64(const double* R, const double* theta, const int* sel,
+template <bool EVEN, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 3) void k_exchange64(const double* R, const double* theta, const int* sel,
                                                           const int* nsel_dev, double* Xp, int N, int GE, int nw, int W,
                                                           int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
                                                           int gridx, int gridy, int gridz) {
-  k_exchange64_body<EVEN>(blockIdx3(), gridDim3(), R, theta, sel, nsel_dev, Xp, N, GE, nw, W, Ktot, s0, s1, ngt_cap, gslot,
+  k_exchange64_body<EVEN, WAVES>(blockIdx3(), gridDim3(), R, theta, sel, nsel_dev, Xp, N, GE, nw, W, Ktot, s0, s1, ngt_cap, gslot,
                           spc, gridx, gridy, gridz);
 }
 
@@ -231,24 +234,32 @@ void launch_exchange64(const DevState& s, const int* sel, int nsel, const int* n
                        hipStream_t st) {
   // chunks of the vectors: at least 8 where there are as many partials, so that the resident
   // workgroups of an XCD (8 walker tiles x 8 chunks, tile_id_at) keep their theta in its L2
-  // while R streams; among those the fewest rounds of the 512 resident workgroups
+  // while R streams; among those the fewest rounds of resident workgroups
   const int gslot = exchange_tile_g(a.n), gt = 64 / a.n, ngt = (int)cdivu(s.GE, gslot), gy = (int)cdivu(nsel, gt);
+  const bool three = gt * a.n <= 48;
+  const int slots = three ? 1024 : 512;   // resident workgroups
   int spc = ngt;
   int64_t best = INT64_MAX;
   for (int nc = std::min(8, ngt); nc <= std::min(64, ngt); ++nc) {
     const int per = (int)cdivu(ngt, nc), z = (int)cdivu(ngt, per);
-    const int64_t cost = (int64_t)cdivu((int64_t)z * gy * nz, 512) * (2 * (int64_t)cdivu((int64_t)per * gslot, gt) + 1);
+    const int64_t cost = (int64_t)cdivu((int64_t)z * gy * nz, slots) * (2 * (int64_t)cdivu((int64_t)per * gslot, gt) + 1);
     if (cost < best) {
       best = cost;
       spc = per;
     }
   }
   const int nx = (int)cdivu(ngt, spc);
-#define AFQ_X64(EVEN_)                                                                                                \
-  afq::glaunch<F_k_exchange64<EVEN_>>((k_exchange64<EVEN_>), dim3((unsigned)(nx * gy * nz)), dim3(X64_NT), 0, st, s.R, s.theta, \
-                                      sel, nsel_dev, xp, s.N, s.GE, nsel, s.W, s.Ktot, a, b, s.ngt_cap, gslot, spc, nx, gy, nz)
-  if (a.n % 2 == 0) AFQ_X64(true);
-  else AFQ_X64(false);
+#define AFQ_X64(EVEN_, WAVES_)                                                                                        \
+  afq::glaunch<F_k_exchange64<EVEN_, WAVES_>>((k_exchange64<EVEN_, WAVES_>), dim3((unsigned)(nx * gy * nz)), dim3(64 * WAVES_), \
+                                              0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel, s.W, s.Ktot, a, b,        \
+                                              s.ngt_cap, gslot, spc, nx, gy, nz)
+  if (a.n % 2 == 0) {
+    if (three) AFQ_X64(true, 3);
+    else AFQ_X64(true, 4);
+  } else {
+    if (three) AFQ_X64(false, 3);
+    else AFQ_X64(false, 4);
+  }
 #undef AFQ_X64
 }
 
