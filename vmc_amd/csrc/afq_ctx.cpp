@@ -841,7 +841,6 @@ int afq_propagate(afq_ctx* c, const double* draws, uint64_t seed, uint64_t step,
   // walkers revived by afq_set_weights get theta and the force bias of their current
   // orbitals before the fields read the force bias
   if (c->fb_stale) ensure_theta(c);
-  afq::launch_zero_counter(s.ncap, c->stream);
   c->last_exact_all = false;
   if (draws) upload(s.draws, draws, (size_t)s.W * s.G, c->stream);
   {
@@ -1903,7 +1902,6 @@ static void batch_enqueue(afq_batch* b, int i, bool qr) {
   // afq::rec_stage() marks the stages the grouped form aligns across systems (the
   // same marks for every system, whatever its kernels)
   afq::rec_stage();
-  afq::launch_zero_counter(s.ncap, st);
   afq::launch_fields(s, nullptr, b->seed + 7919ull * (uint64_t)i, 0, st);
   afq::rec_stage();
   if (s.prec_vhs == AFQ_PREC_FP64) afq::launch_vhs(s, st);

@@ -315,7 +315,6 @@ void launch_debug_gemm_bf16(const double* A, const double* B, float* C, int M, i
                             void* scratch, hipStream_t st);
 void launch_copy_calib(const double* a, double* b, int64_t n, hipStream_t st);
 void launch_fill(double* p, int64_t n, double v, hipStream_t st);
-void launch_zero_counter(unsigned long long* p, hipStream_t st);
 
 void launch_rsplit(const DevState& s, hipStream_t st);
 // pair-wise one-pass exchange: g-tiles per workgroup at most (the partials it keeps in
