@@ -86,21 +86,36 @@ std::vector<double> expm_scaled(const std::vector<double>& H, int N, double s) {
 
 hipEvent_t afq_ctx::ev_get() {
   hipEvent_t e;
+  if (!pool.empty()) {
+    e = pool.back();
+    pool.pop_back();
+    return e;
+  }
   hip_check(hipEventCreate(&e), "hipEventCreate");
   return e;
 }
 void afq_ctx::stage_begin(int st, EvPair& p) {
   if (!timing) return;
-  if (!pool.empty()) { p = pool.back(); pool.pop_back(); }
-  else { p.a = ev_get(); p.b = ev_get(); }
+  if (pending.size() > 4096) resolve();
+  p.a = ev_get();
+  p.first = true;
   p.stage = st;
   hip_check(hipEventRecord(p.a, stream), "hipEventRecord");
 }
+// A marker costs the stream a packet that waits for the work before it, so where nothing lies
+// between two stages one marker ends the first and begins the second.
+void afq_ctx::stage_next(int st, EvPair& p) {
+  if (!timing) return;
+  stage_end(p);
+  p.a = p.b;
+  p.first = false;
+  p.stage = st;
+}
 void afq_ctx::stage_end(EvPair& p) {
   if (!timing) return;
+  p.b = ev_get();
   hip_check(hipEventRecord(p.b, stream), "hipEventRecord");
   pending.push_back(p);
-  if (pending.size() > 4096) resolve();
 }
 void afq_ctx::resolve() {
   for (auto& p : pending) {
@@ -108,7 +123,8 @@ void afq_ctx::resolve() {
     float ms = 0.f;
     hip_check(hipEventElapsedTime(&ms, p.a, p.b), "hipEventElapsedTime");
     stage_ms[p.stage] += ms;
-    pool.push_back(p);
+    if (p.first) pool.push_back(p.a);   // a later pair's a is its predecessor's b
+    pool.push_back(p.b);
   }
   pending.clear();
 }
@@ -131,6 +147,7 @@ struct Stage {
   afq_ctx* c;
   afq_ctx::EvPair p;
   Stage(afq_ctx* c_, int st) : c(c_) { c->stage_begin(st, p); }
+  void next(int st) { c->stage_next(st, p); }   // where nothing is launched between the two stages
   ~Stage() { try { c->stage_end(p); } catch (...) {} }
 };
 
@@ -421,12 +438,10 @@ void refresh_walkers(afq_ctx* c, bool overlaps_from_dets) {
 void ensure_theta(afq_ctx* c) {
   DevState& s = c->s;
   if (!s.theta_stale) return;
-  {
-    Stage t(c, afq::ST_GREEN);
-    afq::launch_green(s, true, c->stream);
-    launch_check("green");
-  }
-  Stage t(c, afq::ST_FB);
+  Stage t(c, afq::ST_GREEN);
+  afq::launch_green(s, true, c->stream);
+  launch_check("green");
+  t.next(afq::ST_FB);
   run_force_bias(s, c->stream);
   launch_check("force_bias");
   s.theta_stale = false;
@@ -669,8 +684,11 @@ int afq_create(const afq_ham* ham, const afq_trial* left, const afq_params* para
 int afq_destroy(afq_ctx* c) {
   if (!c) return AFQ_OK;
   (void)hipStreamSynchronize(c->stream);
-  for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
-  for (auto& p : c->pool) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
+  for (auto& p : c->pending) {
+    if (p.first) (void)hipEventDestroy(p.a);
+    (void)hipEventDestroy(p.b);
+  }
+  for (hipEvent_t e : c->pool) (void)hipEventDestroy(e);
   free_all(c->s);
   free_mlp(c);
   free_cv(c);
@@ -847,45 +865,34 @@ int afq_propagate(afq_ctx* c, const double* draws, uint64_t seed, uint64_t step,
     Stage t(c, afq::ST_FIELDS);
     afq::launch_fields(s, draws ? s.draws : nullptr, seed, step, c->stream);
     launch_check("fields");
-  }
-  {
-    Stage t(c, afq::ST_VHS);
+    t.next(afq::ST_VHS);
     if (s.prec_vhs == AFQ_PREC_FP64) afq::launch_vhs(s, c->stream);
     else afq::launch_vhs_lp(s, s.prec_vhs, c->stream);
     launch_check("vhs");
-  }
-  {
-    Stage t(c, afq::ST_PROP);
-    afq::launch_expmul_pre(s, c->stream);
-  }
-  {
-    Stage t(c, afq::ST_TAYLOR);
+    const bool one = afq::prop_in_one(s);
+    if (!one) {
+      t.next(afq::ST_PROP);
+      afq::launch_expmul_pre(s, c->stream);
+    }
+    t.next(afq::ST_TAYLOR);
     afq::launch_taylor(s, c->stream);
-  }
-  {
-    Stage t(c, afq::ST_PROP);
-    afq::launch_expmul_post(s, c->stream);
+    if (!one) {
+      t.next(afq::ST_PROP);
+      afq::launch_expmul_post(s, c->stream);
+    }
     launch_check("propagate");
-  }
-  {
-    Stage t(c, afq::ST_GREEN);
+    t.next(afq::ST_GREEN);
     // after a comb every walker's overlap matrix is recomputed, propagated or not
     afq::launch_green_pre(s, s.theta_stale, c->stream);
     launch_check("green");
-  }
-  {
-    Stage t(c, afq::ST_WEIGHT);
+    t.next(afq::ST_WEIGHT);
     afq::launch_weight(s, eshift, true, c->stream);
     launch_check("weight");
-  }
-  {
-    Stage t(c, afq::ST_GREEN);
+    t.next(afq::ST_GREEN);
     afq::launch_theta_post(s, c->stream);   // theta of the walkers still alive
     launch_check("theta");
     s.theta_stale = false;
-  }
-  {
-    Stage t(c, afq::ST_FB);
+    t.next(afq::ST_FB);
     run_force_bias(s, c->stream);
     launch_check("force_bias");
   }

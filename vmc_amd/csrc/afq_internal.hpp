@@ -251,6 +251,7 @@ FbPlan fb_plan(int W, int G, int64_t Ktot, int64_t ws_doubles);
 void launch_fields(const DevState& s, const double* draws, uint64_t seed, uint64_t step, hipStream_t st);
 void launch_vhs(const DevState& s, hipStream_t st);
 void launch_propagate(const DevState& s, hipStream_t st);  // E psi, Taylor terms, E acc
+bool prop_in_one(const DevState& s);   // launch_taylor is the whole propagation: the next and launch_expmul_post do nothing
 void launch_expmul_pre(const DevState& s, hipStream_t st);
 void launch_taylor(const DevState& s, hipStream_t st);
 void launch_expmul_post(const DevState& s, hipStream_t st);
@@ -366,8 +367,9 @@ struct afq_ctx {
   std::vector<double> phi[2];
   std::vector<float> dummy;
   // stage timing
-  struct EvPair { hipEvent_t a, b; int stage; };
-  std::vector<EvPair> pending, pool;
+  struct EvPair { hipEvent_t a, b; int stage; bool first; };   // first: a is not another pair's b
+  std::vector<EvPair> pending;
+  std::vector<hipEvent_t> pool;
   double stage_ms[afq::ST_COUNT] = {0};
   bool timing = true;
   // surrogate control variate (its running offset, counts and residual statistics live in
@@ -407,6 +409,7 @@ struct afq_ctx {
   // per-stage device timers (HIP events on the context's stream)
   hipEvent_t ev_get();
   void stage_begin(int st, EvPair& p);
+  void stage_next(int st, EvPair& p);
   void stage_end(EvPair& p);
   void resolve();
 };

@@ -1161,6 +1161,7 @@ static bool prop64(const DevState& s) {
   return s.prec_prop == AFQ_PREC_FP64 && s.taylor_variant != 1 && s.taylor_variant != 2 && prop64_fits(s);
 }
 // psi <- E (sum_{k<=5} V^k / k!) E psi  for every live walker
+bool prop_in_one(const DevState& s) { return prop64(s) || (s.prec_prop != AFQ_PREC_FP64 && prop_fused(s)); }
 void launch_expmul_pre(const DevState& s, hipStream_t st) {
   if (prop64(s)) return;
   if (s.prec_prop != AFQ_PREC_FP64) {
