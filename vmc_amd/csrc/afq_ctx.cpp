@@ -91,7 +91,7 @@ hipEvent_t afq_ctx::ev_get() {
     pool.pop_back();
     return e;
   }
-  hip_check(hipEventCreate(&e), "hipEventCreate");
+  hip_check(hipEventCreateWithFlags(&e, hipEventDisableSystemFence), "hipEventCreate");
   return e;
 }
 void afq_ctx::stage_begin(int st, EvPair& p) {
@@ -103,7 +103,9 @@ void afq_ctx::stage_begin(int st, EvPair& p) {
   hip_check(hipEventRecord(p.a, stream), "hipEventRecord");
 }
 // A marker costs the stream a packet that waits for the work before it, so where nothing lies
-// between two stages one marker ends the first and begins the second.
+// between two stages one marker ends the first and begins the second.  Only its time stamp is
+// read, so it flushes no caches (no system fence).  A block of five steps at N = 10, 128 walkers:
+// two markers a stage 1123 us, shared ones 893, without the fence 794.
 void afq_ctx::stage_next(int st, EvPair& p) {
   if (!timing) return;
   stage_end(p);
