@@ -271,24 +271,6 @@ void ensure_exchange_prec(DevState& s, int prec, hipStream_t st) {
   else if (prec != AFQ_PREC_FP64) ensure_lowprec(s, st);
 }
 
-// Frees the walker buffers of a temporary population that shares the
-// Hamiltonian, trial and bf16 operand buffers of its context.
-void free_all(DevState& s);
-void free_temporary(const DevState& t) {
-  DevState z = t;
-  z.E = z.Lp = z.R = z.mf = nullptr;
-  z.E2 = z.Lp2 = z.P2 = nullptr;   // the context's (a temporary population does not propagate)
-  z.phi[0] = z.phi[1] = z.hphi[0] = z.hphi[1] = nullptr;
-  z.Rb_hi = z.Rb_lo = z.Rf = z.Rf_lo = z.Tb_hi = z.Tb_lo = nullptr;
-  z.fbp = nullptr;
-  z.Lt_hi = z.Lt_lo = z.Fb_hi = z.Fb_lo = nullptr;
-  z.vhs_blk = nullptr;
-  z.Rq8 = nullptr; z.rinv8 = nullptr;   // shared with the context (Tq8/tinv8 are sized by its W)
-  z.Tq8 = nullptr; z.tinv8 = nullptr;
-  z.Vh = z.Vl = z.Ub[0] = z.Ub[1] = z.Ub[2] = z.Dh = z.Dl = nullptr;
-  free_all(z);
-}
-
 // Walker-dependent buffers for a population of W.
 void alloc_walkers(DevState& s) {
   const int64_t W = s.W;
@@ -334,6 +316,44 @@ void upload(double* d, const double* h, size_t n, hipStream_t st) {
 void download(double* h, const double* d, size_t n, hipStream_t st) {
   hip_check(hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, st), "hipMemcpyAsync D2H");
   hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
+}
+
+// Small results to the host: one kernel a result writes them to pinned memory, then one
+// synchronization for all.  hipMemcpyAsync to the caller's pageable memory and a synchronization
+// for each took, on a block of five steps at N = 10, 128 walkers (14 results), 794 us, now 617.  Larger
+// results, which the bus bounds, are copied directly.
+struct Result {
+  void* h;
+  const void* d;
+  size_t n;   // 8-byte words
+};
+constexpr size_t PIN_WORDS = 32768, TMP_KEEP = size_t(64) << 20;
+void readback(afq_ctx* c, std::initializer_list<Result> results) {
+  size_t tot = 0;
+  for (const Result& r : results)
+    if (r.h) tot += r.n;
+  if (tot > PIN_WORDS) {
+    for (const Result& r : results)
+      if (r.h) download(static_cast<double*>(r.h), static_cast<const double*>(r.d), r.n, c->stream);
+    return;
+  }
+  if (tot == 0) return;
+  std::lock_guard<std::mutex> lk(c->pin_mu);
+  if (!c->pin) hip_check(hipHostMalloc(reinterpret_cast<void**>(&c->pin), PIN_WORDS * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
+  size_t o = 0;
+  for (const Result& r : results) {
+    if (!r.h) continue;
+    afq::launch_copy_small(static_cast<const double*>(r.d), c->pin + o, (int)r.n, c->stream);
+    o += r.n;
+  }
+  launch_check("readback");
+  hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+  o = 0;
+  for (const Result& r : results) {
+    if (!r.h) continue;
+    std::memcpy(r.h, c->pin + o, r.n * sizeof(double));
+    o += r.n;
+  }
 }
 
 // Mean-field shifts and propagator constant of DQMCWalker::prepPropR
@@ -696,6 +716,8 @@ int afq_destroy(afq_ctx* c) {
   free_cv(c);
   if (c->rdmAcc) (void)hipFree(c->rdmAcc);
   if (c->rdmPart) (void)hipFree(c->rdmPart);
+  if (c->tmp) (void)hipFree(c->tmp);
+  if (c->pin) (void)hipHostFree(c->pin);
   (void)hipStreamDestroy(c->stream);
   delete c;
   return AFQ_OK;
@@ -821,14 +843,14 @@ int afq_get_walkers(afq_ctx* c, double* dets, double* overlaps, double* weights)
   }
   if (overlaps) {
     std::vector<double> lo(2 * (size_t)s.W);
-    download(lo.data(), s.logO, lo.size(), c->stream);
+    readback(c, {{lo.data(), s.logO, lo.size()}});
     for (int w = 0; w < s.W; ++w) {
       const std::complex<double> o = std::exp(std::complex<double>(lo[2 * w], lo[2 * w + 1]));
       overlaps[2 * w] = o.real();
       overlaps[2 * w + 1] = o.imag();
     }
   }
-  if (weights) download(weights, s.weights, s.W, c->stream);
+  if (weights) readback(c, {{weights, s.weights, (size_t)s.W}});
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }
@@ -901,13 +923,9 @@ int afq_propagate(afq_ctx* c, const double* draws, uint64_t seed, uint64_t step,
   afq::launch_step_stats(s, c->stream);   // sum of the weights, live and propagated counts
   launch_check("step stats");
   c->last_measure_clipped = false;
-  if (factors) download(factors, s.factors, s.W, c->stream);
-  if (n_capped) {
-    unsigned long long v = 0;
-    hip_check(hipMemcpyAsync(&v, s.ncap, sizeof(v), hipMemcpyDeviceToHost, c->stream), "D2H");
-    hip_check(hipStreamSynchronize(c->stream), "sync");
-    *n_capped = (int64_t)v;
-  }
+  unsigned long long capped = 0;
+  readback(c, {{factors, s.factors, (size_t)s.W}, {n_capped ? &capped : nullptr, s.ncap, 1}});
+  if (n_capped) *n_capped = (int64_t)capped;
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }
@@ -998,7 +1016,7 @@ static int measure_cv(afq_ctx* c, double delta, double* eloc) {
   c->cv_nfallback += fallback ? 1 : 0;
   c->last_exact_all = fallback;
   c->last_measure_clipped = !fallback && clip;
-  if (eloc) download(eloc, s.eloc, s.W, st);
+  if (eloc) readback(c, {{eloc, s.eloc, (size_t)s.W}});
   return AFQ_OK;
 }
 
@@ -1026,8 +1044,7 @@ int afq_measure(afq_ctx* c, int32_t mode, double delta, double* eloc, double* ha
   launch_check("energy");
   c->last_exact_all = true;
   c->last_measure_clipped = false;
-  if (eloc) download(eloc, s.eloc, s.W, c->stream);
-  if (ham_ovlp) download(ham_ovlp, s.ho, 4 * (size_t)s.W, c->stream);
+  readback(c, {{eloc, s.eloc, (size_t)s.W}, {ham_ovlp, s.ho, 4 * (size_t)s.W}});
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }
@@ -1036,28 +1053,34 @@ int afq_ham_and_overlap(afq_ctx* c, const double* dets, int32_t ndet, int32_t nc
   if (!c || !dets || !out || ndet <= 0) return c ? fail(c, AFQ_ERR_ARG, "bad arguments") : AFQ_ERR_ARG;
   if (nchol_ene < 0 || nchol_ene > c->s.G) return fail(c, AFQ_ERR_ARG, "nchol_ene out of range");
   AFQ_GUARD_BEGIN
-  // a temporary population of ndet walkers sharing the Hamiltonian buffers
-  DevState t = c->s;
-  t.W = ndet;
-  t.GE = nchol_ene;
-  alloc_walkers(t);
-  t.fbw = t.Sg;
-  t.fbw_doubles = (int64_t)ndet * t.nslots * 64 * 128;
-  try {
-    upload(t.psi, dets, 2 * (size_t)ndet * t.ms, c->stream);
-    afq::launch_fill(t.weights, ndet, 1.0, c->stream);
-    afq::launch_green(t, true, c->stream);
-    afq::launch_logO_from_logdet(t, c->stream);
-    afq::launch_force_bias(t, c->stream);  // FP64: this population is not the one the bf16 buffers cover
-    if (t.GE > 0) afq::launch_exchange(t, nullptr, ndet, c->stream);
-    afq::launch_energy(t, nullptr, ndet, 0.0, c->stream);
-    launch_check("ham_and_overlap");
-    download(out, t.ho, 4 * (size_t)ndet, c->stream);
-  } catch (...) {
-    free_temporary(t);
-    throw;
+  // a temporary population of ndet walkers sharing the Hamiltonian buffers, in one block that the
+  // context keeps up to TMP_KEEP (calls on one context take turns with it)
+  std::lock_guard<std::mutex> lk(c->tmp_mu);
+  DevState t = afq::temporary_population(c->s, ndet, nchol_ene);
+  afq::Carve size{nullptr};
+  afq::carve_population(t, ndet, size);
+  if (size.off > c->tmp_bytes) {
+    if (c->tmp) (void)hipFree(c->tmp);
+    c->tmp = nullptr;
+    c->tmp_bytes = 0;
+    c->tmp = dalloc<unsigned char>(size.off);
+    c->tmp_bytes = size.off;
   }
-  free_temporary(t);
+  afq::Carve cv{c->tmp};
+  afq::carve_population(t, ndet, cv);
+  struct GiveBack {
+    afq_ctx* c;
+    ~GiveBack() {
+      if (c->tmp_bytes <= TMP_KEEP) return;
+      (void)hipFree(c->tmp);
+      c->tmp = nullptr;
+      c->tmp_bytes = 0;
+    }
+  } give_back{c};
+  upload(t.psi, dets, 2 * (size_t)ndet * t.ms, c->stream);
+  afq::launch_temporary(t, c->stream);
+  launch_check("ham_and_overlap");
+  readback(c, {{out, t.ho, 4 * (size_t)ndet}});
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }
@@ -1082,7 +1105,7 @@ int afq_comb(afq_ctx* c, double zeta, double* total_weight) {
     launch_check("comb");
   }
   c->last_exact_all = false;  // the last measurement's per-walker partials refer to the old walkers
-  if (total_weight) download(total_weight, c->s.cum + (c->s.W - 1), 1, c->stream);
+  if (total_weight) readback(c, {{total_weight, c->s.cum + (c->s.W - 1), 1}});
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }
@@ -1668,7 +1691,7 @@ int afq_get_step_stats(afq_ctx* c, afq_step_stats* out) {
   if (!c || !out) return AFQ_ERR_ARG;
   AFQ_GUARD_BEGIN
   double v[afq::STATS_DOUBLES];
-  download(v, c->s.stats, afq::STATS_DOUBLES, c->stream);
+  readback(c, {{v, c->s.stats, afq::STATS_DOUBLES}});
   out->total_weight = v[afq::SS_SUMW];
   out->n_propagated = (int64_t)v[afq::SS_NPROP];
   out->n_live = (int64_t)v[afq::SS_NLIVE];

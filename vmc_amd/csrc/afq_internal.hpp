@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -314,6 +315,7 @@ void launch_rotate_chol(const double* L, const double* phi, double* R, int N, in
 void launch_debug_gemm(const double* A, const double* B, double* C, int M, int N, int K, hipStream_t st);
 void launch_debug_gemm_bf16(const double* A, const double* B, float* C, int M, int N, int K, int passes,
                             void* scratch, hipStream_t st);
+void launch_copy_small(const double* a, double* b, int n, hipStream_t st);   // b may be pinned host memory
 void launch_copy_calib(const double* a, double* b, int64_t n, hipStream_t st);
 void launch_fill(double* p, int64_t n, double v, hipStream_t st);
 
@@ -347,6 +349,72 @@ void launch_vhs_lp(const DevState& s, int prec, hipStream_t st);
 int exchange_tile_g(int n);   // g-blocks per exchange tile for slot size n (0: unsupported)
 int exchange_tile_w(int n);   // walkers per exchange tile
 
+// Hands out 256-byte aligned pieces of one buffer; with base == nullptr it only sizes.
+struct Carve {
+  unsigned char* base;
+  size_t off = 0;
+  template <class T>
+  T* take(size_t n) {
+    off = (off + 255) & ~size_t(255);
+    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+    off += n * sizeof(T);
+    return p;
+  }
+};
+
+// The buffers of a temporary population of ndet walkers that the Green's function,
+// force bias, exchange and energy kernels read or write, carved from c; every other
+// walker buffer of t is null.
+inline void carve_population(DevState& t, int ndet, Carve& c) {
+  const int64_t n = ndet;
+  t.psi = c.take<double>(2 * n * t.ms);
+  t.theta = c.take<double>(2 * n * t.Ktot);
+  t.fb = c.take<double>(2 * n * t.G);
+  t.logO = c.take<double>(2 * n);
+  t.e1 = c.take<double>(2 * n * t.nslots);
+  t.logdet = c.take<double>(2 * n * t.nslots);
+  t.weights = c.take<double>(n);
+  t.Sg = c.take<double>(n * t.nslots * 64 * 128);
+  t.fbw = t.Sg;
+  t.fbw_doubles = n * t.nslots * 64 * 128;
+  t.Xp = c.take<double>(2 * (int64_t)t.nslots * n * t.ngt_cap);
+  t.eloc = c.take<double>(n);
+  t.ho = c.take<double>(4 * n);
+  t.live = c.take<int>(n);
+  t.nlive = c.take<int>(1);
+}
+
+// a population of ndet walkers that shares s's Hamiltonian and trial and no walker buffer
+// (carve_population sets those it needs); ge: Cholesky vectors in the energy
+inline DevState temporary_population(const DevState& s, int ndet, int ge) {
+  DevState t = s;
+  t.factors = t.psi2 = t.theta2 = t.fb2 = t.logO2 = t.e12 = nullptr;
+  t.fields = t.sft = t.P = t.t0 = t.t1 = t.accb = t.draws = t.cum = t.P2 = nullptr;
+  t.idx = t.gfresh = nullptr;
+  t.ncap = nullptr;
+  t.Tb_hi = t.Tb_lo = nullptr;
+  t.fbp = nullptr;
+  t.fbp_rows = 0;
+  t.tb_live = false;
+  t.tb_post = false;
+  t.d_step = nullptr;
+  t.d_eshift = nullptr;
+  t.d_zeta = nullptr;
+  t.graph_mode = false;
+  t.W = ndet;
+  t.GE = ge;
+  return t;
+}
+// (H, overlap) of its walkers into t.ho; FP64: this population is not the one the bf16 buffers cover
+inline void launch_temporary(const DevState& t, hipStream_t st) {
+  launch_fill(t.weights, t.W, 1.0, st);
+  launch_green(t, true, st);
+  launch_logO_from_logdet(t, st);
+  launch_force_bias(t, st);
+  if (t.GE > 0) launch_exchange(t, nullptr, t.W, st);
+  launch_energy(t, nullptr, t.W, 0.0, st);
+}
+
 }  // namespace afq
 
 // One context: one rank's walker population, the Hamiltonian and the trial on one GPU
@@ -356,6 +424,11 @@ struct afq_ctx {
   afq_params params{};
   hipStream_t stream = nullptr;
   std::string err;
+  // a kept block for temporary populations, pinned memory for small results, and who uses them
+  std::mutex tmp_mu, pin_mu;
+  unsigned char* tmp = nullptr;
+  size_t tmp_bytes = 0;
+  double* pin = nullptr;
   bool prepped = false;
   bool have_walkers = false;
   // set by afq_set_weights: a walker it revives may carry a force bias older than its

@@ -3937,6 +3937,9 @@ void launch_debug_gemm_bf16(const double* A, const double* B, float* C, int M, i
     afq::glaunch<F_k_debug_gemm_bf16<1>>(k_debug_gemm_bf16<1>, grid, dim3(256), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp);
 }
 
+void launch_copy_small(const double* a, double* b, int n, hipStream_t st) {
+  afq::glaunch<F_k_copy_calib>(k_copy_calib, dim3(cdivu(n, 256)), dim3(256), 0, st, a, b, (int64_t)n);
+}
 void launch_copy_calib(const double* a, double* b, int64_t n, hipStream_t st) {
   afq::glaunch<F_k_copy_calib>(k_copy_calib, dim3(2048), dim3(256), 0, st, a, b, n);
 }

@@ -1,7 +1,7 @@
 // afq_ham_and_overlap_dev: the local energies of caller-supplied determinants with no
 // device allocation.  afq_ham_and_overlap builds a temporary population (orbitals,
-// theta, overlap matrices, force bias, exchange partials, energies) in memory it
-// allocates and frees on every call; here that population lives in `scratch`, a
+// theta, overlap matrices, force bias, exchange partials, energies) in memory its
+// context allocates; here that population lives in `scratch`, a
 // file-scope device array of AFQ_NOALLOC_SCRATCH_BYTES that every GPU the library runs
 // on holds until the process ends.  The kernels and their order are those of
 // afq_ham_and_overlap, so both entry points return the same numbers.
@@ -55,41 +55,6 @@ unsigned char* scratch_on(int dev, std::string& err) {
   return sl.ptr;
 }
 
-// Hands out 256-byte aligned pieces of one buffer; with base == nullptr it only sizes.
-struct Carve {
-  unsigned char* base;
-  size_t off = 0;
-  template <class T>
-  T* take(size_t n) {
-    off = (off + 255) & ~size_t(255);
-    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
-    off += n * sizeof(T);
-    return p;
-  }
-};
-
-// The buffers of a temporary population of ndet walkers that the Green's function,
-// force bias, exchange and energy kernels read or write, carved from c; every other
-// walker buffer of t is null.
-void carve_population(afq::DevState& t, int ndet, Carve& c) {
-  const int64_t n = ndet;
-  t.psi = c.take<double>(2 * n * t.ms);
-  t.theta = c.take<double>(2 * n * t.Ktot);
-  t.fb = c.take<double>(2 * n * t.G);
-  t.logO = c.take<double>(2 * n);
-  t.e1 = c.take<double>(2 * n * t.nslots);
-  t.logdet = c.take<double>(2 * n * t.nslots);
-  t.weights = c.take<double>(n);
-  t.Sg = c.take<double>(n * t.nslots * 64 * 128);
-  t.fbw = t.Sg;
-  t.fbw_doubles = n * t.nslots * 64 * 128;
-  t.Xp = c.take<double>(2 * (int64_t)t.nslots * n * t.ngt_cap);
-  t.eloc = c.take<double>(n);
-  t.ho = c.take<double>(4 * n);
-  t.live = c.take<int>(n);
-  t.nlive = c.take<int>(1);
-}
-
 int fail_ctx(afq_ctx* c, int code, const std::string& m) {
   c->err = m;
   return code;
@@ -105,29 +70,13 @@ extern "C" int afq_ham_and_overlap_dev(afq_ctx* c, const double* dets_dev, int32
   std::string err;
   unsigned char* base = scratch_on(c->params.device, err);
   if (!base) return fail_ctx(c, AFQ_ERR_DEVICE, err);
-  afq::DevState t = c->s;
-  // no walker buffer of the context is shared: only what carve_population hands out
-  t.factors = t.psi2 = t.theta2 = t.fb2 = t.logO2 = t.e12 = nullptr;
-  t.fields = t.sft = t.P = t.t0 = t.t1 = t.accb = t.draws = t.cum = t.P2 = nullptr;
-  t.idx = t.gfresh = nullptr;
-  t.ncap = nullptr;
-  t.Tb_hi = t.Tb_lo = nullptr;
-  t.fbp = nullptr;
-  t.fbp_rows = 0;
-  t.tb_live = false;
-  t.tb_post = false;
-  t.d_step = nullptr;
-  t.d_eshift = nullptr;
-  t.d_zeta = nullptr;
-  t.graph_mode = false;
-  t.W = ndet;
-  t.GE = nchol_ene;
-  Carve size{nullptr};
-  carve_population(t, ndet, size);
+  afq::DevState t = afq::temporary_population(c->s, ndet, nchol_ene);
+  afq::Carve size{nullptr};
+  afq::carve_population(t, ndet, size);
   if (size.off > (size_t)AFQ_NOALLOC_SCRATCH_BYTES) {
-    Carve one{nullptr};
+    afq::Carve one{nullptr};
     afq::DevState t1 = t;
-    carve_population(t1, 1, one);
+    afq::carve_population(t1, 1, one);
     return fail_ctx(c, AFQ_ERR_ARG,
                     "afq_ham_and_overlap_dev: " + std::to_string(ndet) + " determinants need " +
                         std::to_string(size.off) + " bytes of scratch; the allocation-free entry point has " +
@@ -135,17 +84,12 @@ extern "C" int afq_ham_and_overlap_dev(afq_ctx* c, const double* dets_dev, int32
                         std::to_string((size_t)AFQ_NOALLOC_SCRATCH_BYTES / (one.off + 1024)) +
                         " determinants of this shape)");
   }
-  Carve cv{base};
-  carve_population(t, ndet, cv);
+  afq::Carve cv{base};
+  afq::carve_population(t, ndet, cv);
   const hipStream_t st = c->stream;
   hipError_t e = hipMemcpyAsync(t.psi, dets_dev, 2 * sizeof(double) * (size_t)ndet * t.ms, hipMemcpyDeviceToDevice, st);
   if (e != hipSuccess) return fail_ctx(c, AFQ_ERR_DEVICE, std::string("hipMemcpyAsync: ") + hipGetErrorString(e));
-  afq::launch_fill(t.weights, ndet, 1.0, st);
-  afq::launch_green(t, true, st);
-  afq::launch_logO_from_logdet(t, st);
-  afq::launch_force_bias(t, st);   // FP64, as afq_ham_and_overlap
-  if (t.GE > 0) afq::launch_exchange(t, nullptr, ndet, st);
-  afq::launch_energy(t, nullptr, ndet, 0.0, st);
+  afq::launch_temporary(t, st);
   e = hipGetLastError();
   if (e != hipSuccess) return fail_ctx(c, AFQ_ERR_DEVICE, std::string("ham_and_overlap_dev: ") + hipGetErrorString(e));
   e = hipMemcpyAsync(out_dev, t.ho, 4 * sizeof(double) * (size_t)ndet, hipMemcpyDeviceToDevice, st);
