@@ -1308,24 +1308,25 @@ void launch_propagate(const DevState& s, hipStream_t st) {
 //  1. k_overlap: S = Phi_s^T psi for every walker of a slot as one GEMM over the
 //     W * 2n real columns (FP64 MFMA), into Sg[w][slot] (64 x 128 doubles each);
 //  2. k_invert: S^-1 and log det S per (walker, slot) by Gauss-Jordan elimination with
-//     partial pivoting, the matrix held in registers (lane = row, wave q = complex
-//     columns CPW q .. CPW q + CPW - 1), so a workgroup needs only 3 KB of LDS;
+//     partial pivoting, the matrix held in registers (lane = row; one wave's columns, or
+//     CPW q .. CPW q + CPW - 1 for wave q of several);
 //  3. k_theta: theta = psi S^-1 (FP64 MFMA, S^-1 held in LDS) and the one-body
 //     partial e1 = sum theta o (h1 Phi).
 // In a propagation step 1-2 run before the weight update (the overlap ratio needs
 // log det S of every propagated walker) and 3 after it, for the walkers still alive.
-// one step of a wave maximum of 64-bit keys (hi, lo) by a DPP move: a lane of the rows in
-// RM takes the key of the lane CTRL names when that one is larger
+// one step of a wave maximum by a DPP move: a lane of the rows in RM takes the key of the lane
+// CTRL names when that one is larger
 template <int CTRL, int RM>
-__device__ __forceinline__ void dpp_max_step(unsigned& hi, unsigned& lo) {
-  const unsigned oh = (unsigned)__builtin_amdgcn_update_dpp((int)hi, (int)hi, CTRL, RM, 0xF, false);
-  const unsigned ol = (unsigned)__builtin_amdgcn_update_dpp((int)lo, (int)lo, CTRL, RM, 0xF, false);
-  const bool take = oh > hi || (oh == hi && ol > lo);
-  hi = take ? oh : hi;
-  lo = take ? ol : lo;
+__device__ __forceinline__ unsigned dpp_max_step(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, RM, 0xF, false);
+  return max(v, o);
 }
 
-template <int CPW>
+// x[0 .. CPW) are a wave's columns, in register slots that rotate: the wave that holds column k
+// has it in slot 0, and its update moves every slot down one (the results simply go to the
+// registers of the slot below) with column k's successor at the top, so that the step needs no
+// register index and is not unrolled over k.
+template <int CPW, bool MULTI>
 __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim_, GreenArgs a) {
   __shared__ cplx colb[2][GN_MAX];
   __shared__ cplx pvs[GN_MAX];
@@ -1335,7 +1336,8 @@ __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim
   if (a.fresh && si == 0 && threadIdx.x == 0) a.fresh[w] = take ? 1 : 0;
   if (!take) return;
   const Slot sl = si == 0 ? a.s0 : a.s1;
-  const int n = sl.n, tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
+  const int n = sl.n, tid = threadIdx.x, lane = tid & 63;
+  const int q = !MULTI ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
   double* S = a.Sg + ((int64_t)w * a.nslots + si) * SG_MAT;
   cplx x[CPW];
 #pragma unroll
@@ -1346,59 +1348,79 @@ __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim
   }
   bool used = lane >= n;
   int myk = 0;
-  // step k = CPW o + c: column k lives in wave o at slot c; the slot loop is unrolled,
-  // so every choice that depends on the slot is made at compile time
-  for (int o = 0; o * CPW < n; ++o) {
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const int k = CPW * o + c;
-      if (k >= n) continue;   // wave-uniform
-      if (q == o) colb[c & 1][lane] = x[c];
+  for (int k = 0, o = 0, c = 0; k < n; ++k, ++c) {
+    if (MULTI && c == CPW) {
+      c = 0;
+      ++o;
+    }
+    cplx f = x[0];
+    if (MULTI) {
+      if (q == o) colb[k & 1][lane] = x[0];
       __syncthreads();
-      const cplx f = colb[c & 1][lane];
-      // pivot: the unused row of largest |f|^2, ties to the lower row.  |f|^2 >= 0, so its
-      // bits order like its value; the low 7 bits carry 64 - row (rows whose |f|^2 agree to
-      // 2^-45 relative count as tied), and a used row has key 0.  The maximum over the wave
-      // by DPP moves (no LDS round trips): pairs, quads, half rows, rows, then rows 1 and 3
-      // take rows 0 and 2, and row 3 takes row 1, so lane 63 ends with it.
-      const unsigned long long key =
-          used ? 0ull
-               : ((unsigned long long)__double_as_longlong(f.re * f.re + f.im * f.im) & ~0x7Full) |
-                     (unsigned long long)(64 - lane);
-      unsigned khi = (unsigned)(key >> 32), klo = (unsigned)key;
-      dpp_max_step<0xB1, 0xF>(khi, klo);    // quad_perm [1,0,3,2]
-      dpp_max_step<0x4E, 0xF>(khi, klo);    // quad_perm [2,3,0,1]
-      dpp_max_step<0x141, 0xF>(khi, klo);   // row_half_mirror
-      dpp_max_step<0x140, 0xF>(khi, klo);   // row_mirror
-      dpp_max_step<0x142, 0xA>(khi, klo);   // row_bcast:15 into rows 1 and 3
-      dpp_max_step<0x143, 0xC>(khi, klo);   // row_bcast:31 into rows 2 and 3
-      const int p = 64 - (int)(__builtin_amdgcn_readlane((int)klo, 63) & 0x7F);
-      const cplx pv = colb[c & 1][p];
-      // 1 / pv = conj(pv) / |pv|^2 (one division; the pivots of an overlap matrix are
-      // far from the range where |pv|^2 would overflow or underflow)
-      const double rn = 1.0 / (pv.re * pv.re + pv.im * pv.im);
-      const cplx pinv{pv.re * rn, -pv.im * rn};
-      if (lane == p) { used = true; myk = k; }
-      if (tid == 0) {
-        pk[k] = p;
-        pvs[k] = pv;
-      }
-      // every other row minus (f_i / pv) times row p; row p itself keeps its scale
-      // until the end (every row is divided by its own pivot after the last step, so
-      // the update of a column is one complex multiply-add).  The stored column k
-      // turns into column p of the inverse (in place): 1 in row p (divided by pv at
-      // the end) and -f_i / pv elsewhere.
-      cplx g = cmul(f, pinv);
-      if (lane == p) g = cplx{0.0, 0.0};
+      f = colb[k & 1][lane];
+    }
+    // pivot: the unused row of largest |f|^2, ties to the lower row.  |f|^2 >= 0, so its
+    // high word orders like its value; its low 7 bits carry 64 - row (rows whose |f|^2 agree to
+    // 2^-13 relative count as tied, and a pivot that close to the largest serves as well), and a
+    // used row has key 0.  The maximum over the wave
+    // by DPP moves (no LDS round trips): pairs, quads, half rows, rows, then rows 1 and 3
+    // take rows 0 and 2, and row 3 takes row 1, so lane 63 ends with it.
+    unsigned key = used ? 0u
+                        : ((unsigned)__double2hiint(f.re * f.re + f.im * f.im) & ~0x7Fu) | (unsigned)(64 - lane);
+    key = dpp_max_step<0xB1, 0xF>(key);    // quad_perm [1,0,3,2]
+    key = dpp_max_step<0x4E, 0xF>(key);    // quad_perm [2,3,0,1]
+    key = dpp_max_step<0x141, 0xF>(key);   // row_half_mirror
+    key = dpp_max_step<0x140, 0xF>(key);   // row_mirror
+    key = dpp_max_step<0x142, 0xA>(key);   // row_bcast:15 into rows 1 and 3
+    key = dpp_max_step<0x143, 0xC>(key);   // row_bcast:31 into rows 2 and 3
+    const int p = 64 - (int)(__builtin_amdgcn_readlane((int)key, 63) & 0x7F);
+    const cplx pv{readlane_f64(f.re, p), readlane_f64(f.im, p)};
+    // 1 / pv = conj(pv) / |pv|^2 (one division; the pivots of an overlap matrix are
+    // far from the range where |pv|^2 would overflow or underflow)
+    const double rn = 1.0 / (pv.re * pv.re + pv.im * pv.im);
+    const cplx pinv{pv.re * rn, -pv.im * rn};
+    if (lane == p) { used = true; myk = k; }
+    if (tid == 0) {
+      pk[k] = p;
+      pvs[k] = pv;
+    }
+    // every other row minus (f_i / pv) times row p; row p itself keeps its scale
+    // until the end (every row is divided by its own pivot after the last step, so
+    // the update of a column is one complex multiply-add).  The stored column k
+    // turns into column p of the inverse (in place): 1 in row p (divided by pv at
+    // the end) and -f_i / pv elsewhere.
+    cplx g = cmul(f, pinv);
+    if (lane == p) g = cplx{0.0, 0.0};
+    // four columns at a time, all broadcasts first: a use right behind its broadcast, and the
+    // second FMA of an element right behind the first, would wait for it
+    auto update = [&](auto from, auto to) {
 #pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        const cplx xp{readlane_f64(x[j].re, p), readlane_f64(x[j].im, p)};
-        cplx nx{x[j].re - g.re * xp.re + g.im * xp.im, x[j].im - g.re * xp.im - g.im * xp.re};
-        if (j == c && q == o) nx = lane == p ? cplx{1.0, 0.0} : cplx{-g.re, -g.im};
-        x[j] = nx;
+      for (int j0 = 0; j0 < CPW; j0 += 4) {
+        cplx xp[4], t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (from(j0 + j) < CPW) xp[j] = cplx{readlane_f64(x[from(j0 + j)].re, p), readlane_f64(x[from(j0 + j)].im, p)};
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (from(j0 + j) < CPW) {
+            const cplx v = x[from(j0 + j)];
+            t[j] = cplx{v.re - g.re * xp[j].re, v.im - g.re * xp[j].im};
+          }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (from(j0 + j) < CPW) x[to(j0 + j)] = cplx{t[j].re + g.im * xp[j].im, t[j].im - g.im * xp[j].re};
       }
+    };
+    if (!MULTI || q == o) {
+      update([](int j) { return j + 1; }, [](int j) { return j; });
+      x[CPW - 1] = lane == p ? cplx{1.0, 0.0} : cplx{-g.re, -g.im};
+    } else {
+      update([](int j) { return j; }, [](int j) { return j; });
     }
   }
+  // how far this wave's slots have rotated: slot j holds its column (j + rot) mod CPW
+  const int rot = max(0, min(n - CPW * q, CPW));
   __syncthreads();
   if (lane < n) {
     // row p_k (this lane's, k = myk) divided by its pivot
@@ -1412,7 +1434,7 @@ __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim
   if (lane < n) {
 #pragma unroll
     for (int j = 0; j < CPW; ++j) {
-      const int col = CPW * q + j;
+      const int col = CPW * q + (j + rot < CPW ? j + rot : j + rot - CPW);
       if (col < n) {
         const int lc = pk[col];
         S[myk * SG_LD + 2 * lc] = x[j].re;
@@ -1425,46 +1447,56 @@ __device__ __forceinline__ void k_invert_body(const uint3 bid_, const uint3 gdim
     cplx l = lane < n ? clog(pvs[lane]) : cplx{0.0, 0.0};
     const double ld_re = wave_sum(l.re);
     double ld_im = wave_sum(l.im);
-    unsigned long long seen = 0ull;
-    int cycles = 0;
-    for (int k = 0; k < n; ++k) {
-      if (seen >> k & 1ull) continue;
-      ++cycles;
-      for (int t = k; t >= 0 && t < n && !(seen >> t & 1ull); t = pk[t]) seen |= 1ull << t;
-    }
-    if ((n - cycles) & 1) ld_im += M_PI;
+    // the sign by the inversions of k -> p_k, each lane counting its own
+    int inv = 0;
+    const int mine = lane < n ? pk[lane] : 0;
+    for (int k = 0; k + 1 < n; ++k) inv += lane > k && lane < n && pk[k] > mine ? 1 : 0;
+    const unsigned long long odd = __ballot(inv & 1);
+    if (__popcll(odd) & 1) ld_im += M_PI;
     if (lane == 0) {
       a.logdet[2 * ((int64_t)w * a.nslots + si)] = ld_re;
       a.logdet[2 * ((int64_t)w * a.nslots + si) + 1] = ld_im;
     }
   }
 }
-template <int CPW>
+// waves a SIMD holds: 4 CPW registers for the columns and about 50 more
+constexpr int inv_occ(int cpw) { return cpw <= 12 ? 4 : cpw <= 24 ? 3 : 2; }
+template <int CPW, bool MULTI>
 struct F_k_invert {
-  static constexpr int NT = 256, OCC = CPW == 16 ? 3 : 4;
+  static constexpr int NT = MULTI ? 256 : 64, OCC = inv_occ(CPW);
   static constexpr bool HAS_OCC = true;
   template <class... A>
   __device__ __forceinline__ void operator()(const uint3 b, const uint3 g, A... a) const {
-    k_invert_body<CPW>(b, g, a...);
+    k_invert_body<CPW, MULTI>(b, g, a...);
   }
 };
-template <int CPW>
-__global__ __launch_bounds__(256, CPW == 16 ? 3 : 4) void k_invert(GreenArgs a) {
-  k_invert_body<CPW>(blockIdx3(), gridDim3(), a);
+template <int CPW, bool MULTI>
+__global__ __launch_bounds__(MULTI ? 256 : 64, inv_occ(CPW)) void k_invert(GreenArgs a) {
+  k_invert_body<CPW, MULTI>(blockIdx3(), gridDim3(), a);
 }
 
-// CPW columns a wave and as many waves as the slots' columns fill: a wave's work per step is
-// its columns whether they hold data or not (2048 matrices of n = 20: 59 us as three waves of
-// 8 columns, 99 as four of 16)
+// Bound by VALU issue, of which a step's pivot search and division are about as much as the
+// update of 8 columns, and with few matrices by a step's latency.  So one wave takes a whole
+// matrix up to n = 32, without barriers, where there are more matrices than half the SIMDs (2048
+// of n = 20: 48 us, three waves of 8 columns 58; 24 systems of n = 4 to 24, 256 walkers: 161 us
+// against 213), and with fewer several waves share one (32 of n = 20: 17 us, one wave 21).  Past n = 32 four waves
+// of 16 columns: 1.02 ms for 8192 matrices of n = 60 and 90 us for 512 (two of 32: 1.01 and 140).
 static void launch_invert(const GreenArgs& a, hipStream_t st) {
   const int nmax = std::max(a.s0.n, a.nslots > 1 ? a.s1.n : 0);
   const dim3 grid(a.W, a.nslots);
-  if (nmax <= 16)
-    afq::glaunch<F_k_invert<4>>(k_invert<4>, grid, dim3(64 * cdivu(nmax, 4)), 0, st, a);
-  else if (nmax <= 32)
-    afq::glaunch<F_k_invert<8>>(k_invert<8>, grid, dim3(64 * cdivu(nmax, 8)), 0, st, a);
-  else
-    afq::glaunch<F_k_invert<16>>(k_invert<16>, grid, dim3(64 * cdivu(nmax, 16)), 0, st, a);   // 4 waves: faster than 8 at n = 60
+  const bool few = (int64_t)a.W * a.nslots <= 512 && !g_recorder;   // a grouped launch fills the chip
+#define AFQ_INV(CPW, MULTI) \
+  afq::glaunch<F_k_invert<CPW, MULTI>>((k_invert<CPW, MULTI>), grid, dim3(MULTI ? 64 * cdivu(nmax, CPW) : 64), 0, st, a)
+  if (nmax > 32) AFQ_INV(16, true);
+  else if (few && nmax > 16) AFQ_INV(8, true);
+  else if (few) AFQ_INV(4, true);
+  else if (nmax <= 8) AFQ_INV(8, false);
+  else if (nmax <= 12) AFQ_INV(12, false);
+  else if (nmax <= 16) AFQ_INV(16, false);
+  else if (nmax <= 20) AFQ_INV(20, false);
+  else if (nmax <= 24) AFQ_INV(24, false);
+  else AFQ_INV(32, false);
+#undef AFQ_INV
 }
 
 static GreenArgs green_args(const DevState& s, bool all) {
