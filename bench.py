@@ -190,8 +190,8 @@ def stage_rooflines(spec, path, n_exact):
             # the exact subset of the control variate; the HBM counter summary keeps its
             # dispatches apart from the unclipped shadow measurements on the same kernel
             extra["profile_row"] = "k_exchange (exact subset)"
-        add("exchange", "k_exchange (FP64 MFMA)", exchange_flops(spec, n_exact),
-            8.0 * G * ms + 16.0 * ms * n_exact, 1, "fp64", symbol="k_exchange", walkers=n_exact, **extra)
+        add("exchange", "k_exchange64 (FP64 MFMA)", exchange_flops(spec, n_exact),
+            8.0 * G * ms + 16.0 * ms * n_exact, 1, "fp64", symbol="k_exchange64", walkers=n_exact, **extra)
     else:
         nmax3 = max(nsp)
         if 12 < nmax3 <= 64 and (Np + 31) // 32 * 32 <= 448:
@@ -231,13 +231,18 @@ def stage_rooflines(spec, path, n_exact):
     tay_bytes = Wp * (16.0 * N * N + 4 * 16.0 * ms) * 5
     if path.get("fb_vhs_prec", "fp64") == "fp64":
         wide = ncol > 64
-        add("taylor", "k_taylor (5 complex V t products, FP64 MFMA)", Wp * 40.0 * N * N * ncol, tay_bytes, 5,
-            "fp64", symbol=("void k_taylor<%s>" % ("true" if N % 2 == 0 else "false")) if wide
-            else "void k_vmul<64, 128, 2, 2>")
+        if st.get("onebody", 0.0) <= 0.0:
+            # both one-body factors and the five products in one kernel: V once per product, the orbitals once
+            add("taylor", "k_prop64 (E (sum_k V^k/k!) E psi, fused, FP64 MFMA)", Wp * (40.0 + 8.0) * N * N * ncol,
+                Wp * (5 * 16.0 * N * N + 32.0 * ms), 1, "fp64", symbol="k_prop64")
+        else:
+            add("taylor", "k_taylor (5 complex V t products, FP64 MFMA)", Wp * 40.0 * N * N * ncol, tay_bytes, 5,
+                "fp64", symbol=("void k_taylor<%s>" % ("true" if N % 2 == 0 else "false")) if wide
+                else "void k_vmul<64, 128, 2, 2>")
         add("force_bias", "k_fb64 (FP64 MFMA)", Wl * 4.0 * ncol * N * G, 8.0 * G * ms + Wl * 16.0 * (ms + G),
             1, "fp64", symbol="k_fb64")
-        add("vhs", "k_vhs (FP64 MFMA)", Wp * 4.0 * T * G, 8.0 * G * T + Wp * 16.0 * (G + N * N), 1, "fp64",
-            symbol="k_vhs")
+        add("vhs", "k_vhs64 (FP64 MFMA)", Wp * 4.0 * T * G, 8.0 * G * T + Wp * 16.0 * (G + N * N), 1, "fp64",
+            symbol="k_vhs64")
     else:
         Nq = (N + 15) // 16 * 16
         vb, ub = 8.0 * Nq * N, 8.0 * ncol * Nq
@@ -275,9 +280,9 @@ def stage_rooflines(spec, path, n_exact):
             Wp * (40.0 + 32.0) * ms, 2 * len(nsp), "bf16", symbol="void k_onebody_split<%d>" % mi, passes=3)
     # S = Phi^T psi and its inverse for the walkers propagated, theta = psi S^-1 for the
     # walkers still alive
-    add("green", "k_overlap + k_invert + k_theta_r (FP64 MFMA + Gauss-Jordan)",
+    add("green", "k_overlap + k_invert + k_theta (FP64 MFMA + Gauss-Jordan)",
         sum(Wp * (4 * n * n * N + 16 * n ** 3) + Wl * 8 * N * n * n for n in nsp), (Wp + Wl) * 16.0 * ms, 1,
-        "fp64", symbol="k_theta_r")
+        "fp64", symbol="k_theta")
     return out
 
 
