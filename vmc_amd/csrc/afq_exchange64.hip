@@ -9,9 +9,9 @@ namespace afq {
 
 static inline unsigned cdivu(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
-// One workgroup (four waves) takes gt = 64 / n walkers of a slot and a chunk of the
-// Cholesky vectors, gt at a time: the tile's rows are (vector, i), at most 64, its columns
-// (walker, j), at most 64 complex ones, 16 for each wave.  Both operands go from global
+// One workgroup (WAVES of them, 4 or 3) takes gt = 64 / n walkers of a slot and a chunk of the
+// Cholesky vectors, gt at a time: the tile's rows are (vector, i), at most 16 WAVES, its columns
+// (walker, j), at most 16 WAVES complex ones, 16 for each wave.  Both operands go from global
 // memory straight into MFMA registers, NS - 1 K steps of 4 ahead: one 16-byte load of a lane
 // holds re and im of a theta column (the B operands of two MFMA tiles), and for even n two
 // rows of R_g (the A operands of two tiles: rows 2 l of 32 in one, 2 l + 1 in the other; for
@@ -236,6 +236,10 @@ void launch_exchange64(const DevState& s, const int* sel, int nsel, const int* n
   // workgroups of an XCD (8 walker tiles x 8 chunks, tile_id_at) keep their theta in its L2
   // while R streams; among those the fewest rounds of resident workgroups
   const int gslot = exchange_tile_g(a.n), gt = 64 / a.n, ngt = (int)cdivu(s.GE, gslot), gy = (int)cdivu(nsel, gt);
+  // gt n rows and columns fill 44 to 48 at n = 22 to 24 and 33 to 48 with one walker a tile: the
+  // fourth wave would have no columns there, and a tile of 48 leaves registers and LDS for four
+  // workgroups on a CU instead of two.  N = 100, G = 400, 1024 walkers, n = 23: 4.75 ms with four
+  // waves, 3.73 with three; n = 24 4.68 and 3.65; N = 300, n = 40 and 45, 128 walkers 9.3 and 8.4.
   const bool three = gt * a.n <= 48;
   const int slots = three ? 1024 : 512;   // resident workgroups
   int spc = ngt;
