@@ -288,8 +288,9 @@ int afq_get_one_rdm(afq_ctx* ctx, int32_t spin_summed, double* rdm, double* cumu
 
 /* Per-stage device time (ms) accumulated since the last reset, AFQ_NSTAGES
  * entries in the order force_bias, fields, vhs, one-body (E psi), green, weight,
- * ortho, exchange, comb, taylor (the five V t products), exchange_lp (the
- * reduced-precision exchange of the AFQ_SURR_EXCHANGE surrogate). */
+ * ortho, exchange, comb, taylor (the five V t products; the whole propagation where
+ * one kernel does it, and one-body is then 0), exchange_lp (the reduced-precision
+ * exchange of the AFQ_SURR_EXCHANGE surrogate). */
 #define AFQ_NSTAGES 11
 int afq_stage_times(afq_ctx* ctx, double* ms, int32_t reset);
 
