@@ -19,13 +19,21 @@ static inline unsigned cdivu(int64_t a, int64_t b) { return (unsigned)((a + b - 
 // workgroup share the R lines in the vector L1, and without staging the K loop has no
 // barrier.  f then goes to LDS and the sum runs over i <= j (off-diagonal pairs count
 // twice), so that every element of f is read once.  A group of tpb threads keeps the same
-// (vector, walker) place of the tile for the whole chunk and accumulates in registers; the
-// chunk's sum goes to the first of the chunk's partials and zeros to the others.
+// (vector, walker) place of the tile and accumulates in registers.
+//
+// The vectors fall into units of uv (a multiple of gt), a chunk being whole units, and at a unit's
+// end one wave adds up its sum into its own partial (the walker's further partials are zero).  Units
+// depend on n and on the vectors in the energy alone, never on how many walkers are taken together,
+// which decides only how many units a chunk has: so a walker's exchange is the same to the last bit in
+// any company.  Against one sum for a whole chunk: N = 300, 60+60, 256 walkers 48.2 against 48.0 ms,
+// N = 100, 20+20, 1024 walkers 2.82 both, N = 160, 40+40, 128 walkers 4.66 against 4.48 (units divide
+// the chunks less evenly), N = 51, 13+11, 256 walkers 0.165 against 0.151; with the sum as a tree over
+// the workgroup's threads behind barriers 2.91 at N = 100.
 //
 // Bound by FP64 MFMA issue.  N = 300, 60+60, G = 1200, 256 walkers: 53.4 ms on the 128 x 128
-// LDS-staged kernel before, 47.8 now (56 TFLOP/s useful, 64 with the padding of 60 to 64;
+// LDS-staged kernel before, 48.2 now (55 TFLOP/s useful, 64 with the padding of 60 to 64;
 // 46.0 of it the K loops, timed without the pair sums).  N = 100, 20+20, G = 400, 1024
-// walkers: 3.8 -> 2.86 ms (47 TFLOP/s; K loops 2.54).  A form with LDS stages of both
+// walkers: 3.8 -> 2.82 ms (47 TFLOP/s; K loops 2.54).  A form with LDS stages of both
 // operands took 56 and 3.3 ms (two 8-byte LDS reads per MFMA), one with 8-byte global loads
 // per tile 49.2 and 3.06.  NS = 6 against 4: equal at N = 100 and 300, 3% faster on systems of
 // N = 20 to 120.
@@ -35,21 +43,31 @@ struct X64Shape {
   static constexpr int LDF = 2 * ROWS + 2;   // 16-byte rows; transposed 16-byte reads of 16 lanes on 64 banks
 };
 typedef double __attribute__((ext_vector_type(2), aligned(8))) x64_pair;   // two rows of R, 8-byte aligned
+// x of the lane that DPP control CTRL names
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const int hi = __double2hiint(x), lo = __double2loint(x);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false));
+}
 template <bool EVEN, int WAVES>
 __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* theta,
                                                   const int* sel, const int* nsel_dev, double* Xp, int N, int GE, int nw,
-                                                  int W, int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
+                                                  int W, int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int nt, int uv, int nu, int upc,
                                                   int gridx, int gridy, int gridz) {
   constexpr int NS = 6, NT = X64Shape<WAVES>::NT, LDF = X64Shape<WAVES>::LDF;
   __shared__ __attribute__((aligned(16))) double lds[X64Shape<WAVES>::ROWS * LDF];
+  __shared__ double2 red[NT];
+  __shared__ int walker[16];
   const TileId tl = tile_id_at(bid_.x, gridx, gridy, gridz, 8);
   const Slot sl = tl.z == 0 ? s0 : s1;
   const int n = sl.n, gt = 64 / n, w0 = tl.y * gt, nrow = gt * n;
   if (nsel_dev) nw = *nsel_dev;
   if (w0 >= nw) return;
-  const int ga = tl.x * spc * gslot, gb = min(GE, ga + spc * gslot);   // this chunk's vectors
+  const int ga = tl.x * upc * uv, gb = min(GE, ga + upc * uv);   // this chunk's vectors, units tl.x upc .. + upc - 1
   const int tid = threadIdx.x, lane = tid & 63, cl = lane & 15, kh = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < gt) walker[tid] = w0 + tid >= nw ? -1 : sel ? sel[w0 + tid] : w0 + tid;
   const bool busy = 16 * wave < nrow;   // this wave's columns hold data
   // rows 32 .. nrow (gt n > 32 always): as two tiles, or as one where at most 16 (row 32 + cl)
   const int rest = nrow - 32;
@@ -115,15 +133,24 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
     }
   };
   // pair sums: threads [b tpb, (b + 1) tpb) take block b = (vector b / gt, walker b % gt) of a tile
-  const int tpb = NT / (gt * gt);
+  const int tpb = NT / (gt * gt), rtpb = 65536 / tpb + 1;
   const int blk = tid / tpb, lt = tid - blk * tpb, pg = blk / gt, pw = blk - pg * gt;
   // units (p, t): rows p and n - 1 - p share the n + 1 pairs i <= j
   const int np = (n + 1) >> 1, sp = tpb / (n + 1), stt = tpb - sp * (n + 1);
+  int place = pw << 24 | pg << 16 | (lt / (n + 1)) << 8 | lt % (n + 1);   // one register through the K loops
+  // the lane's number asked for again, so that no register holds it or an address through the K loops
+  auto lane_again = [] {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+  };
   double accr = 0.0, acci = 0.0;
   rows(ga);
 #pragma unroll
   for (int i = 0; i + 1 < NS; ++i) load(i, i);
-  for (int g0 = ga; g0 < gb; g0 += gt) {
+  int unit = tl.x * upc, ub = min(gb, ga + uv);   // the unit at hand and its end
+  for (int g0 = ga; g0 < gb;) {
+    const int gn = min(g0 + gt, ub);   // the next tile's first vector
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -145,7 +172,7 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
         step(i);
       }
     // the next tile's first steps are in flight during the pair sums
-    rows(g0 + gt);
+    rows(gn);
 #pragma unroll
     for (int i = 0; i + 1 < NS; ++i) load(i, i);
     if (busy) {
@@ -163,9 +190,10 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
         }
     }
     __syncthreads();
-    if (pg < gt && g0 + pg < gb) {
-      const double* F = lds + pg * n * LDF + pw * 2 * n;
-      int p = lt / (n + 1), t = lt - p * (n + 1);
+    asm volatile("" : "+v"(place));
+    if ((place >> 16 & 255) < min(gt, gn - g0)) {
+      const double* F = lds + (place >> 16 & 255) * n * LDF + (place >> 24) * 2 * n;
+      int p = place >> 8 & 255, t = place & 255;
       while (p < np) {
         const bool first = t < n - p;
         const int i = first ? p : n - 1 - p, j = first ? p + t : t - 1;   // second row: j = i + t - (n - p)
@@ -181,34 +209,50 @@ __device__ __forceinline__ void k_exchange64_body(const uint3 bid_, const uint3 
         if (t > n) { t -= n + 1; ++p; }
       }
     }
+    if (gn == ub) {
+      red[64 * wave + lane_again()] = double2{accr, acci};
+      accr = acci = 0.0;
+    }
     __syncthreads();
-  }
-  // sums of the thread groups (a tree over the group), then of a walker's vectors in order
-  lds[2 * tid] = accr;
-  lds[2 * tid + 1] = acci;
-  int off = 1;
-  while (2 * off < tpb) off *= 2;
-  for (; off > 0; off >>= 1) {
-    __syncthreads();
-    if (lt < off && lt + off < tpb) {
-      lds[2 * tid] += lds[2 * (tid + off)];
-      lds[2 * tid + 1] += lds[2 * (tid + off) + 1];
+    g0 = gn;
+    if (g0 < ub) continue;
+    ub = min(gb, ub + uv);
+    // the unit's sum by one wave while the others go on: 2^sh lanes a walker take its gt tpb threads'
+    // sums in turn (at most 7 each), then a tree over the lanes.  (red is written again only behind the
+    // next tile's barriers.)
+    if (wave == 0) {
+      const int lq = lane_again();
+      int sh = 6;
+      while (gt << sh > 64) --sh;
+      const int q = lq >> sh, sub = lq & ((1 << sh) - 1), ne = q < gt ? gt * tpb : 0;
+      double xr = 0.0, xi = 0.0;
+#pragma unroll
+      for (int i = 0; i < 7; ++i) {
+        const int e = sub + (i << sh), g = e * rtpb >> 16;   // e / tpb for e < 256
+        if (e < ne) {
+          const double2 x = red[(g * gt + q) * tpb + e - g * tpb];
+          xr += x.x;
+          xi += x.y;
+        }
+      }
+      if (sh >= 5) {
+        for (int off = 1 << (sh - 1); off >= 16; off >>= 1) {
+          xr += __shfl_xor(xr, off, 64);
+          xi += __shfl_xor(xi, off, 64);
+        }
+      }
+      if (sh >= 4) xr += dpp_f64<0x140>(xr), xi += dpp_f64<0x140>(xi);   // row_mirror
+      if (sh >= 3) xr += dpp_f64<0x141>(xr), xi += dpp_f64<0x141>(xi);   // row_half_mirror
+      xr += dpp_f64<0x4E>(xr), xi += dpp_f64<0x4E>(xi);                  // quad_perm [2,3,0,1]
+      xr += dpp_f64<0xB1>(xr), xi += dpp_f64<0xB1>(xi);                  // quad_perm [1,0,3,2]
+      const int w = sub == 0 && q < gt ? walker[q] : -1;
+      if (w >= 0) {
+        double2* o = reinterpret_cast<double2*>(Xp) + ((int64_t)tl.z * W + w) * ngt_cap;
+        o[unit] = double2{xr, xi};
+        for (int t = unit + nu; t < nt; t += nu) o[t] = double2{0.0, 0.0};
+      }
     }
-  }
-  __syncthreads();
-  if (tid < gt && w0 + tid < nw) {
-    double xr = 0.0, xi = 0.0;
-    for (int g = 0; g < gt; ++g) {
-      xr += lds[2 * (g * gt + tid) * tpb];
-      xi += lds[2 * (g * gt + tid) * tpb + 1];
-    }
-    const int w = sel ? sel[w0 + tid] : w0 + tid;
-    double* o = Xp + 2 * (((int64_t)tl.z * W + w) * ngt_cap);
-    const int t0 = tl.x * spc, t1 = min((GE + gslot - 1) / gslot, t0 + spc);
-    for (int t = t0; t < t1; ++t) {
-      o[2 * t] = t == t0 ? xr : 0.0;
-      o[2 * t + 1] = t == t0 ? xi : 0.0;
-    }
+    ++unit;
   }
 }
 template <bool EVEN, int WAVES>
@@ -223,40 +267,43 @@ struct F_k_exchange64 {
 template <bool EVEN, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 3) void k_exchange64(const double* R, const double* theta, const int* sel,
                                                           const int* nsel_dev, double* Xp, int N, int GE, int nw, int W,
-                                                          int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int gslot, int spc,
+                                                          int64_t Ktot, Slot s0, Slot s1, int ngt_cap, int nt, int uv, int nu, int upc,
                                                           int gridx, int gridy, int gridz) {
-  k_exchange64_body<EVEN, WAVES>(blockIdx3(), gridDim3(), R, theta, sel, nsel_dev, Xp, N, GE, nw, W, Ktot, s0, s1, ngt_cap, gslot,
-                          spc, gridx, gridy, gridz);
+  k_exchange64_body<EVEN, WAVES>(blockIdx3(), gridDim3(), R, theta, sel, nsel_dev, Xp, N, GE, nw, W, Ktot, s0, s1, ngt_cap, nt, uv, nu,
+                          upc, gridx, gridy, gridz);
 }
 
 // slots a and b (b of a's size; nz = 1: a alone), partials at xp
 void launch_exchange64(const DevState& s, const int* sel, int nsel, const int* nsel_dev, double* xp, Slot a, Slot b, int nz,
                        hipStream_t st) {
-  // chunks of the vectors: at least 8 where there are as many partials, so that the resident
-  // workgroups of an XCD (8 walker tiles x 8 chunks, tile_id_at) keep their theta in its L2
-  // while R streams; among those the fewest rounds of resident workgroups
-  const int gslot = exchange_tile_g(a.n), gt = 64 / a.n, ngt = (int)cdivu(s.GE, gslot), gy = (int)cdivu(nsel, gt);
+  // units of the vectors: whole tiles, no more units than there are partials, and 64 at most (a unit
+  // costs about 900 cycles of one wave, 3 % with units of two tiles at N = 100)
+  const int gslot = exchange_tile_g(a.n), gt = 64 / a.n, nt = (int)cdivu(s.GE, gslot), gy = (int)cdivu(nsel, gt);
+  const int u1 = (int)cdivu(gslot, gt) * gt, uv = u1 * (int)cdivu(cdivu(s.GE, u1), 64), nu = (int)cdivu(s.GE, uv);
   // gt n rows and columns fill 44 to 48 at n = 22 to 24 and 33 to 48 with one walker a tile: the
   // fourth wave would have no columns there, and a tile of 48 leaves registers and LDS for four
   // workgroups on a CU instead of two.  N = 100, G = 400, 1024 walkers, n = 23: 4.75 ms with four
   // waves, 3.73 with three; n = 24 4.68 and 3.65; N = 300, n = 40 and 45, 128 walkers 9.3 and 8.4.
   const bool three = gt * a.n <= 48;
   const int slots = three ? 1024 : 512;   // resident workgroups
-  int spc = ngt;
+  // chunks of units: at least 8 where there are as many, so that the resident workgroups of an XCD
+  // (8 walker tiles x 8 chunks, tile_id_at) keep their theta in its L2 while R streams; among those
+  // the fewest rounds of resident workgroups
+  int upc = nu;
   int64_t best = INT64_MAX;
-  for (int nc = std::min(8, ngt); nc <= std::min(64, ngt); ++nc) {
-    const int per = (int)cdivu(ngt, nc), z = (int)cdivu(ngt, per);
-    const int64_t cost = (int64_t)cdivu((int64_t)z * gy * nz, slots) * (2 * (int64_t)cdivu((int64_t)per * gslot, gt) + 1);
+  for (int nc = std::min(8, nu); nc <= nu; ++nc) {
+    const int per = (int)cdivu(nu, nc), z = (int)cdivu(nu, per);
+    const int64_t cost = (int64_t)cdivu((int64_t)z * gy * nz, slots) * (2 * (int64_t)per * (uv / gt) + 1);
     if (cost < best) {
       best = cost;
-      spc = per;
+      upc = per;
     }
   }
-  const int nx = (int)cdivu(ngt, spc);
+  const int nx = (int)cdivu(nu, upc);
 #define AFQ_X64(EVEN_, WAVES_)                                                                                        \
   afq::glaunch<F_k_exchange64<EVEN_, WAVES_>>((k_exchange64<EVEN_, WAVES_>), dim3((unsigned)(nx * gy * nz)), dim3(64 * WAVES_), \
                                               0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel, s.W, s.Ktot, a, b,        \
-                                              s.ngt_cap, gslot, spc, nx, gy, nz)
+                                              s.ngt_cap, nt, uv, nu, upc, nx, gy, nz)
   if (a.n % 2 == 0) {
     if (three) AFQ_X64(true, 3);
     else AFQ_X64(true, 4);
