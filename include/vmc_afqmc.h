@@ -388,8 +388,8 @@ int afq_set_exchange_variant(afq_ctx* ctx, int32_t variant);
 int afq_set_exchange_chunks(afq_ctx* ctx, int32_t chunks);
 /* FP64 exchange kernel (no counterpart in the reference): 0 (default) 64-row x 64-complex-
  * column tiles whose operands go straight from memory to registers, for slots of at least
- * 4 electrons (below: as 2); 128 x 128 tiles through LDS: 1 the element-loader engine (two
- * barriers per stage), 2 the pointer-loader engine (double-buffered stages). */
+ * 4 electrons (below: as 2, with 8 waves); 128 x 128 tiles through LDS: 1 the element-loader
+ * engine (two barriers per stage), 2 the pointer-loader engine (double-buffered stages, 4 waves). */
 int afq_set_exchange64_variant(afq_ctx* ctx, int32_t variant);
 /* Split-BF16 VHS tile (no counterpart in the reference): 0 128 (walker, component) rows
  * by one 16 x 8 block of V, 64-deep single-buffered stages; 1 256 rows, eight waves,

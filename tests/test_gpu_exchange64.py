@@ -67,3 +67,11 @@ def test_exchange_matches_numpy(case):
 ], ids=lambda c: "N%d_%d_%d_G%d_W%d" % c[:5])
 def test_exchange_three_waves_matches_numpy(case):
     test_exchange_matches_numpy(case)
+
+
+@pytest.mark.parametrize("case", [
+    # slots of one to three electrons, on both sides of a 128-row tile of vectors and walkers
+    (4, 1, 1, 129, 130, 129), (7, 2, 1, 65, 129, 60), (9, 2, 2, 64, 64, 64), (10, 3, 2, 43, 43, 42), (10, 3, 3, 85, 90, 85),
+], ids=lambda c: "N%d_%d_%d_G%d_W%d" % c[:5])
+def test_exchange_of_few_electrons_matches_numpy(case):
+    test_exchange_matches_numpy(case)

@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # N, na, nb, G, RHF trial and walkers
+    (12, 3, 2, 50, False),      # fewer than four electrons
     (20, 4, 4, 90, False),      # 16 walkers and vectors a tile
     (30, 11, 8, 130, False),    # slots of different size
     (47, 23, 17, 163, False),   # odd; three waves for one spin

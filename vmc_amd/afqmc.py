@@ -199,7 +199,7 @@ class Context:
 
     def set_exchange64_variant(self, variant):
         """FP64 exchange kernel: 0 (default) operands straight into registers (from 4 electrons a slot,
-        below that as 2), 1 element loaders, 2 pointer-loader engine with 4 waves."""
+        below that as 2 with 8 waves), 1 element loaders, 2 pointer-loader engine with 4 waves."""
         L = lib()
         L.afq_set_exchange64_variant.argtypes = [C.c_void_p, C.c_int32]
         self._chk(L.afq_set_exchange64_variant(self.ptr, int(variant)), "afq_set_exchange64_variant")

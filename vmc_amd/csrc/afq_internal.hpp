@@ -169,7 +169,7 @@ struct DevState {
   // (0: by shape)
   int xc_chunks = 0;
   // FP64 exchange kernel: 0 by shape (k_exchange64 from 4 electrons a slot up, else
-  // k_exchange2), 1 k_exchange (element loaders), 2 k_exchange2
+  // k_exchange2 with 8 waves), 1 k_exchange (element loaders), 2 k_exchange2 with 4 waves
   int xc64_variant = 0;
   // split-BF16 force bias: one workgroup per slot and FP64 combine (true, default), or
   // both slots in one workgroup

@@ -1932,7 +1932,7 @@ __global__ __launch_bounds__(256, 2) void k_exchange(const double* R, const doub
 }
 
 // k_exchange on the pointer-loader engine (MmaF64P: double-buffered stages, no index
-// arithmetic per element): 128 x 128 tiles over 4 waves (WN = 2).
+// arithmetic per element): 128 x 128 tiles over 4 (WN = 2) or 8 waves (WN = 4).
 template <int WN>
 __device__ __forceinline__ void k_exchange2_body(const uint3 bid_, const uint3 gdim_, const double* R, const double* theta, const int* sel,
                                                           const int* nsel_dev, double* Xp, int N, int GE, int nw,
@@ -2015,8 +2015,12 @@ void launch_exchange(const DevState& s, const int* sel, int nsel, hipStream_t st
     if (s.xc64_variant == 1)
       afq::glaunch<F_k_exchange>(k_exchange, grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel, s.W,
                                  s.Ktot, a, b, s.ngt_cap, ngt, gy, nz);
-    else
+    else if (s.xc64_variant == 2)
       afq::glaunch<F_k_exchange2<2>>((k_exchange2<2>), grid, dim3(256), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel,
+                                     s.W, s.Ktot, a, b, s.ngt_cap, ngt, gy, nz);
+    else   // up to 3 electrons, eight waves: n = 1, 2, 3 at N = 50, G = 200, 1024 walkers 139, 78 and 83 us (four waves 163,
+           // 90 and 85); n = 3 at N = 100, G = 400, 4096 walkers 656 us (731), at N = 12, G = 48, 256 walkers 51 (62)
+      afq::glaunch<F_k_exchange2<4>>((k_exchange2<4>), grid, dim3(512), 0, st, s.R, s.theta, sel, nsel_dev, xp, s.N, s.GE, nsel,
                                      s.W, s.Ktot, a, b, s.ngt_cap, ngt, gy, nz);
   };
   if (s.nslots == 1 || s.slot[1].n == s.slot[0].n) {
