@@ -200,7 +200,8 @@ int afq_measure(afq_ctx* ctx, int32_t mode, double delta, double* eloc, double* 
 /* E_L of arbitrary determinants against the left trial (init-time helper used
  * for the reference energy and the Cholesky truncation search,
  * DQMC/MixedEstimator.cpp:352-384).  dets: ndet determinants in serial layout;
- * out: ndet x {E*O, O} complex. */
+ * out: ndet x {E*O, O} complex.  FP64 results of a determinant or a walker (these, the
+ * force bias, the exact energies) do not depend on how many others one call takes. */
 int afq_ham_and_overlap(afq_ctx* ctx, const double* dets, int32_t ndet,
                         int32_t nchol_ene, double* out);
 

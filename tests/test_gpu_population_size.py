@@ -61,3 +61,38 @@ def test_exchange_energy_in_any_company(case):
     weights = rng.integers(0, 2, len(every)).astype(float)
     got = exchange(every, weights)
     assert np.array_equal(got[weights != 0.0], want[weights != 0.0])
+
+
+@pytest.mark.parametrize("case", CASES + [
+    # the force bias' sum over (orbital, electron) pairs: too short to divide; divided, where theta is
+    # larger than the overlap matrices; more vectors than an overlap matrix holds
+    (7, 2, 2, 20, False), (150, 40, 36, 230, False), (20, 3, 3, 4200, True),
+], ids=lambda c: "N%d_%d_%d_G%d%s" % (c[:4] + ("_rhf" if c[4] else "",)))
+def test_force_bias_and_energies_in_any_company(case):
+    """Force biases between populations; energies and overlaps also between populations and the calls that
+    evaluate given determinants."""
+    h, dets, rng = system(*case)
+    keep = h.nchol - 1
+
+    def walkers(pick, weights=None):
+        ctx = Context(h, len(pick), case[4])
+        ctx.set_nchol_ene(keep)
+        ctx.set_walkers(dets[pick], weights=weights)
+        fb, (energies, ho) = ctx.force_bias(), ctx.measure()
+        ctx.close()
+        return fb, energies, ho
+
+    every = np.arange(COUNTS[-1])
+    fb, energies, ho = walkers(every)
+    ctx = Context(h, 1, case[4])
+    for count in COUNTS:
+        for first in (0, 7):
+            pick = every[first:first + count]
+            if count < COUNTS[-1]:
+                got = walkers(pick)
+                assert np.array_equal(got[0], fb[pick]) and np.array_equal(got[1], energies[pick])
+            assert np.array_equal(ctx.ham_and_overlap(dets[pick], keep).ravel(), np.asarray(ho).reshape(len(every), -1)[pick].ravel())
+    ctx.close()
+    weights = rng.integers(0, 2, len(every)).astype(float)
+    got, live = walkers(every, weights), weights != 0.0
+    assert np.array_equal(got[0][live], fb[live]) and np.array_equal(got[1][live], energies[live])

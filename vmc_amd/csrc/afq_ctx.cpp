@@ -616,6 +616,7 @@ int afq_create(const afq_ham* ham, const afq_trial* left, const afq_params* para
     }
     s.Ktot = 0;
     for (int q = 0; q < s.nslots; ++q) s.Ktot += (int64_t)N * s.slot[q].n;
+    s.fbo = afq::fb_order(G, s.Ktot, s.nslots);
     s.Np = (N + 7) / 8 * 8;
     s.ctot = 0;
     for (int q = 0; q < s.nslots; ++q) s.ctot += 2 * s.slot[q].n;

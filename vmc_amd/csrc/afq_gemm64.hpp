@@ -1,16 +1,13 @@
 // FP64 MFMA block product with 16-byte operand loads, for the contractions whose
-// operands lie in memory in one of three ways:
+// operands lie in memory in one of two ways:
 //   StageC  complex rows, K contiguous: element k of row pair (2w, 2w + 1) is one
 //           (re, im) double2, so one 16-byte load feeds a real row and its imaginary twin
 //   StageK  real rows, K contiguous: one 16-byte load holds two K of a row
-//   StageR  rows contiguous at each k (element (k, row) at base + k * stride + row):
-//           one 16-byte load holds two rows of a k
 // One stage is BK = 16 deep, double-buffered in LDS: stage s + 1 goes global ->
 // registers before stage s is multiplied and registers -> LDS after it, one barrier a
 // stage.  The K order inside a stage is 8 s + 2 (lane / 16) + {0, 1}, so that a lane of
-// a K-contiguous operand reads the operands of two MFMAs with one ds_read_b128; rows of
-// 18 doubles put the 16 lanes of such a read on 64 different banks, and a row pitch of
-// 8 mod 16 doubles does so for StageR's 8-byte reads.
+// an operand reads the operands of two MFMAs with one ds_read_b128; rows of 18 doubles put
+// the 16 lanes of such a read on 64 different banks.
 #pragma once
 #include "afq_device.hpp"
 
@@ -106,7 +103,9 @@ struct StageK {
   }
 };
 
-// C += A B for a BM x BN tile over K in [k0, kend), k0 a multiple of 16; waves WM x WN.
+// C += A B for a BM x BN tile over K in [k0, kend), k0 a multiple of 16; waves WM x WN.  At the
+// end of every ku of K (a multiple of 16) and of the last, shorter one, unit(acc) is called, and
+// acc starts from zero again.
 template <class SA, class SB, int BM, int BN, int WAVES_M, int WAVES_N>
 struct Gemm64 {
   static constexpr int NT = 64 * WAVES_M * WAVES_N;
@@ -120,13 +119,18 @@ struct Gemm64 {
     const int wave = threadIdx.x >> 6;
     wm = wave / WAVES_N;
     wn = wave % WAVES_N;
+    clear();
+  }
+  __device__ __forceinline__ void clear() {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
   }
-  __device__ __forceinline__ void run(SA& sa, SB& sb, int k0, int kend, double* lds) {
+  template <class U>
+  __device__ __forceinline__ void run(SA& sa, SB& sb, int k0, int kend, double* lds, int ku, const U& unit) {
     if (k0 >= kend) return;
+    int uend = k0 + ku;
     sa.fetch(k0, kend);
     sb.fetch(k0, kend);
     sa.put(lds);
@@ -163,6 +167,11 @@ struct Gemm64 {
         sa.put(lds + buf * STAGE);
         sb.put(lds + buf * STAGE + SA::SIZE);
       }
+      if (!more || k + G64_BK == uend) {
+        unit(acc);
+        clear();
+        uend += ku;
+      }
       __syncthreads();
     }
   }
@@ -170,13 +179,13 @@ struct Gemm64 {
   __device__ __forceinline__ int row(int i, int r) const { return wm * WM + i * 16 + (lane >> 4) + 4 * r; }
   __device__ __forceinline__ int col(int j) const { return wn * WN + j * 16 + (lane & 15); }
   template <class EP>
-  __device__ __forceinline__ void store(const EP& ep) const {
+  __device__ __forceinline__ void store(const f64x4 (&v)[TM][TN], const EP& ep) const {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ep(row(i, r), col(j), acc[i][j][r]);
+        for (int r = 0; r < 4; ++r) ep(row(i, r), col(j), v[i][j][r]);
   }
 };
 

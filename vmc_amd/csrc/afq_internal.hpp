@@ -39,6 +39,9 @@ enum StatSlot {
 };
 constexpr int STATS_DOUBLES = 32;
 
+// order of an FP64 force bias sum over k: units of ku (a multiple of 16), chunks of s units
+struct FbOrder { int ku, s; };
+
 struct DevState {
   // sizes
   int N = 0, na = 0, nb = 0, G = 0, GE = 0, W = 0;
@@ -90,9 +93,10 @@ struct DevState {
   // FP64 force bias: partial sums over chunks of K.  Not a buffer of its own: it borrows
   // one that nothing reads between the Green's function and the end of the force bias,
   // the larger of Sg (S^-1 is used up by theta) and theta2 (live inside a comb only);
-  // a temporary population borrows Sg, whichever entry point made it, so that all of
-  // them split K alike
+  // a temporary population borrows Sg, whichever entry point made it.  fbo is the order of
+  // the sum, which is the same for all of them
   double* fbw = nullptr; int64_t fbw_doubles = 0;
+  FbOrder fbo{};
   double* Xp = nullptr;      // nslots x W x ngt complex exchange partials
   int ngt_cap = 0;
   double* eloc = nullptr;    // W
@@ -245,10 +249,10 @@ void launch_risk_split(const DevState& s, const double* ej, double risk, RiskSor
 
 // kernel launchers (afq_kernels.hip)
 void launch_force_bias(const DevState& s, hipStream_t st);   // afq_force_bias.hip
-// the split of the FP64 force bias of W walkers: the 32 x 64 or the 64 x 64 tile, and
-// nz chunks of kchunk (a multiple of 16) of the Ktot products
-struct FbPlan { bool small; int nz, kchunk; };
-FbPlan fb_plan(int W, int G, int64_t Ktot, int64_t ws_doubles);
+// the workgroups of the FP64 force bias of a population: the 32 x 64 or the 64 x 64 tile, nz of them
+// along K with m units each, np parts in the workspace, each a unit or (whole) a chunk
+struct FbSplit { bool small, whole; int m, nz, np; double cost; };
+FbOrder fb_order(int G, int64_t Ktot, int nslots);
 void launch_fields(const DevState& s, const double* draws, uint64_t seed, uint64_t step, hipStream_t st);
 void launch_vhs(const DevState& s, hipStream_t st);
 void launch_propagate(const DevState& s, hipStream_t st);  // E psi, Taylor terms, E acc
