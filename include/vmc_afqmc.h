@@ -361,15 +361,15 @@ int afq_debug_cv_force_position(afq_ctx* ctx, int32_t position);
 
 /* ---------------------------------------------------------------- tuning
  * Propagation-kernel autotuner (no counterpart in the reference): times the kernel
- * variants of the context's propagation precision on its current walkers (without
- * changing them) and keeps the fastest.  FP64, the five Taylor products: 1 = 64 x 128
- * real tiles, 2 = 128 x 128 complex tiles; where the fused FP64 kernel applies (N <= 384)
- * and is faster than both, the context keeps that one, and choice names the better of
- * these two.  Split BF16, the whole propagation
- * E (sum V^k/k!) E: 1 = 128-orbital and 2 = 160-orbital row tiles with the one-body
- * factors and each Taylor step as separate kernels, 3 = one fused kernel per block of
- * columns (N <= 384 only).  choice (nullable) receives the variant; ms3 (nullable, 3
- * entries) the times in ms per propagation (0 for a variant not tried). */
+ * variants of the context's whole propagation E (sum V^k/k!) E in its precision on its
+ * current walkers (without changing them) and keeps the fastest.  FP64: 1 = 64 x 128 real
+ * tiles, 2 = 128 x 128 complex tiles, and, where it applies (N <= 384), the fused kernel.
+ * Split BF16: 1 = 128-orbital and 2 = 160-orbital row tiles with the one-body factors and
+ * each Taylor step as separate kernels, 3 = one fused kernel per block of columns (N <= 384
+ * only).  choice (nullable) receives the variant; in FP64 it names the better of 1 and 2
+ * also where the fused kernel is kept, and handing it to afq_set_taylor_variant then turns
+ * that kernel off (0 keeps it on).  ms3 (nullable, 3 entries): the times in ms per
+ * propagation (0 for a variant not tried, and for the third in FP64). */
 int afq_autotune(afq_ctx* ctx, int32_t* choice, double* ms3);
 /* 0: by shape (default: the fused kernel where it applies), 1, 2 or 3: the variants
  * named at afq_autotune (3 falls back to the shape rule where N > 384 or in FP64, whose

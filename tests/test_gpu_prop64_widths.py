@@ -4,12 +4,14 @@ whole and with a short last tile, one block and several, against the separate on
 A wide block is only taken by a population that fills the chip, so 256 walkers.  The bound is that of
 test_gpu_prop64: seven products of at most 2N terms, each rounding to 7 * 2N * 2^-53 of the orbitals'
 scale (6e-13 at N = 384) in either order of summation."""
+import ctypes as C
+
 import numpy as np
 import pytest
 from test_gpu_prop64 import set_variant, system
 
 from vmc_amd.abi import HamArrays
-from vmc_amd.afqmc import Context
+from vmc_amd.afqmc import Context, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +84,33 @@ def test_every_width_matches_separate_kernels(case):
     assert np.max(np.abs(out[0] - out[2])) <= 2e-12 * scale
     dead = weights == 0.0
     assert np.array_equal(out[0][dead], dets[dead]) and not np.any(np.all(out[0][~dead] == dets[~dead], axis=1))
+
+
+def test_autotuner_times_whole_propagations():
+    """Every variant is timed over the same work, both one-body factors included: against the stage timers of
+    steps taken with it (the factors are a tenth of it or more, half of which the comparison asks for)."""
+    h = system(100, 24, 20, False, seed=5)
+    ctx = Context(h, 1024, False)
+    ctx.prep_prop(h.phi_up, h.phi_dn, 0.01)
+    ctx.set_walkers_uniform(h.serial_det(h.phi_up, h.phi_dn))
+    stages = []
+    for variant in (1, 2):
+        assert set_variant(ctx, variant) == 0
+        times = []
+        for step in range(6):
+            ctx.set_weights(np.ones(1024))
+            ctx.stage_times()
+            ctx.propagate(None, 0.0, seed=1, step=step)
+            times.append([ctx.stage_times(reset=False)[k] for k in ("taylor", "onebody")])
+        stages.append(np.median(times[1:], axis=0))
+    ctx.set_weights(np.ones(1024))
+    choice, ms = C.c_int32(0), (C.c_double * 3)()
+    assert lib().afq_autotune(ctx.ptr, C.byref(choice), ms) == 0
+    ctx.stage_times()
+    ctx.propagate(None, 0.0, seed=1, step=9)
+    kept = ctx.stage_times()
+    ctx.close()
+    print("whole propagations", list(ms), "taylor, one-body", stages, "kept", kept["taylor"] + kept["onebody"])
+    for t, (taylor, onebody) in zip(ms, stages):
+        assert t >= taylor + 0.5 * onebody
+    assert kept["taylor"] + kept["onebody"] <= 1.1 * min(ms[0], ms[1])

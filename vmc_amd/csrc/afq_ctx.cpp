@@ -1766,11 +1766,11 @@ int afq_sync(afq_ctx* c) {
 }  // extern "C"
 
 // ---------------------------------------------------------------- autotuner
-// Times the alternative tile shapes of the Taylor products (k_vmul's 64 x 128 real
-// tiles against k_taylor's 128 x 128-complex tiles) on this context's current
-// walkers and keeps the faster one; in FP64 the fused k_prop64, where it applies, is kept
-// over both when its whole propagation takes less than their Taylor products alone.  The
-// products only write Taylor scratch, so the walker state is unchanged.
+// Times the variants of the whole propagation (both one-body factors and the series) on
+// this context's current walkers and keeps the fastest: in FP64 k_vmul's 64 x 128 real tiles
+// and k_taylor's 128 x 128-complex tiles, each between the one-body products, and, where it
+// applies, the fused k_prop64; in split BF16 the two row tiles and the fused kernel.  The
+// results go to the scratch t1, so the walkers stay as they are.
 int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   if (!c) return AFQ_ERR_ARG;
   if (!c->prepped || !c->have_walkers) return fail(c, AFQ_ERR_STATE, "afq_prep_prop and afq_set_walkers first");
@@ -1779,41 +1779,21 @@ int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   hipEvent_t a, b;
   hip_check(hipEventCreate(&a), "event");
   hip_check(hipEventCreate(&b), "event");
-  double best = 1e300;
-  int pick = 1;
+  double ms[4] = {0.0, 0.0, 0.0, 0.0};   // of variants 1 .. 3
   const int keep = s.taylor_variant;
-  bool fused64 = false;
-  // split BF16: the whole propagation (both one-body factors and the series) into the
-  // scratch t1, so the walkers stay as they are; FP64: the five Taylor products
   const bool split = s.prec_prop != AFQ_PREC_FP64;
-  const int nv = split && afq::prop_fused_fits(s) ? 3 : 2;
-  if (ms_out) ms_out[2] = 0.0;
-  auto run = [&]() {
-    if (split) afq::launch_prop_split_to(s, s.t1, c->stream);
-    else afq::launch_taylor(s, c->stream);
-  };
+  const int nv = (split ? afq::prop_fused_fits(s) : afq::prop64_fits(s)) ? 3 : 2;
   try {
     for (int v = 1; v <= nv; ++v) {
       s.taylor_variant = v;
-      run();  // warm
+      afq::launch_propagate_to(s, s.t1, c->stream);  // warm
       hip_check(hipEventRecord(a, c->stream), "record");
-      for (int r = 0; r < 3; ++r) run();
+      for (int r = 0; r < 3; ++r) afq::launch_propagate_to(s, s.t1, c->stream);
       hip_check(hipEventRecord(b, c->stream), "record");
       hip_check(hipEventSynchronize(b), "sync");
-      float ms = 0.f;
-      hip_check(hipEventElapsedTime(&ms, a, b), "elapsed");
-      if (ms_out) ms_out[v - 1] = ms / 3.0;
-      if (ms < best) { best = ms; pick = v; }
-    }
-    if (!split && afq::prop64_fits(s)) {
-      afq::launch_prop64(s, s.t1, c->stream);  // warm
-      hip_check(hipEventRecord(a, c->stream), "record");
-      for (int r = 0; r < 3; ++r) afq::launch_prop64(s, s.t1, c->stream);
-      hip_check(hipEventRecord(b, c->stream), "record");
-      hip_check(hipEventSynchronize(b), "sync");
-      float ms = 0.f;
-      hip_check(hipEventElapsedTime(&ms, a, b), "elapsed");
-      fused64 = ms < best;
+      float t = 0.f;
+      hip_check(hipEventElapsedTime(&t, a, b), "elapsed");
+      ms[v] = t / 3.0;
     }
   } catch (...) {
     s.taylor_variant = keep;
@@ -1823,8 +1803,13 @@ int afq_autotune(afq_ctx* c, int32_t* choice, double* ms_out) {
   }
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
-  s.taylor_variant = fused64 ? 0 : pick;
+  int pick = ms[2] < ms[1] ? 2 : 1;
+  if (split && nv == 3 && ms[3] < ms[pick]) pick = 3;
+  // FP64: choice and ms3 name the two tile shapes; the fused kernel is the shape rule's own (0)
+  s.taylor_variant = !split && nv == 3 && ms[3] < ms[pick] ? 0 : pick;
   if (choice) *choice = pick;
+  if (ms_out)
+    for (int v = 1; v <= 3; ++v) ms_out[v - 1] = split || v < 3 ? ms[v] : 0.0;
   return AFQ_OK;
   AFQ_GUARD_END(c)
 }

@@ -263,7 +263,7 @@ void launch_expmul_post(const DevState& s, hipStream_t st);
 bool prop_fused_fits(const DevState& s);                              // k_prop_split handles N
 bool prop64_fits(const DevState& s);                                  // k_prop64 handles N (afq_prop64.hip)
 void launch_prop64(const DevState& s, double* dst, hipStream_t st);   // the fused FP64 propagation, result in dst
-void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st);  // split path, result in dst
+void launch_propagate_to(const DevState& s, double* dst, hipStream_t st);   // the whole propagation, result in dst
 void launch_green(const DevState& s, bool all_walkers, hipStream_t st);
 void launch_green_pre(const DevState& s, bool all_walkers, hipStream_t st);   // S, S^-1, log det S
 void launch_theta_post(const DevState& s, hipStream_t st);                   // theta, e1 of the live walkers

@@ -1144,9 +1144,7 @@ static void launch_prop_fused(const DevState& s, const double* src, double* dst,
   else prop_split_m<3>(s, ct, src, dst, st);
 }
 static void launch_taylor_split(const DevState& s, hipStream_t st);
-// The split path's whole propagation with the result in dst (psi itself in a step;
-// scratch when the autotuner times it)
-void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st) {
+static void launch_prop_split_to(const DevState& s, double* dst, hipStream_t st) {
   if (prop_fused(s)) {
     launch_prop_fused(s, s.psi, dst, st);
     return;
@@ -1282,19 +1280,33 @@ void launch_taylor(const DevState& s, hipStream_t st) {
     double* t = src; src = dst; dst = t;
   }
 }
-void launch_expmul_post(const DevState& s, hipStream_t st) {
-  if (prop64(s)) return;
-  if (s.prec_prop != AFQ_PREC_FP64) {
-    if (!prop_fused(s)) launch_onebody_split(s, s.accb, s.psi, 1, st);
-    return;
-  }
+// the closing FP64 one-body factor: dst <- E acc
+static void expmul_post_to(const DevState& s, double* dst, hipStream_t st) {
   const int64_t ws = 2 * s.ms;
   for (int d = 0; d < s.ndets_prop; ++d) {
     const int n = s.det_n[d];
     const int gx = (int)cdivu((int64_t)s.W * 2 * n, EX_BN), gy = (int)cdivu(s.N, EX_BM);
     const double* E = (s.uints && d == 1) ? s.E2 : s.E;
-    afq::glaunch<F_k_expmul>(k_expmul, dim3(gx * gy), dim3(256), 0, st, E, s.accb, s.psi, nullptr, s.weights,
+    afq::glaunch<F_k_expmul>(k_expmul, dim3(gx * gy), dim3(256), 0, st, E, s.accb, dst, nullptr, s.weights,
                        s.N, n, s.W, ws, 2 * s.det_off[d], 1, gx, gy);
+  }
+}
+void launch_expmul_post(const DevState& s, hipStream_t st) {
+  if (prop64(s)) return;
+  if (s.prec_prop == AFQ_PREC_FP64) expmul_post_to(s, s.psi, st);
+  else if (!prop_fused(s)) launch_onebody_split(s, s.accb, s.psi, 1, st);
+}
+// The whole propagation (both one-body factors and the series) of the context's variant
+// with the result in dst, which may be t1: the walkers stay as they are
+void launch_propagate_to(const DevState& s, double* dst, hipStream_t st) {
+  if (s.prec_prop != AFQ_PREC_FP64) {
+    launch_prop_split_to(s, dst, st);
+  } else if (prop64(s)) {
+    launch_prop64(s, dst, st);
+  } else {
+    launch_expmul_pre(s, st);
+    launch_taylor(s, st);
+    expmul_post_to(s, dst, st);
   }
 }
 void launch_propagate(const DevState& s, hipStream_t st) {
